@@ -37,33 +37,43 @@ __device__ __forceinline__ float half_bits_to_f32(uint16_t hbits) {
   return static_cast<float>(__builtin_bit_cast(_Float16, hbits));
 }
 
-// Quantise one group of 32 fp32 values; returns the fp16 scale bits.
-__device__ __forceinline__ uint16_t q6_quantize_group(const float* x, uint8_t* codes24) {
-  float amax = 0.f;
-#pragma unroll
-  for (int e = 0; e < kGroup; ++e) amax = fmaxf(amax, fabsf(x[e]));
+// The fp16 scale bits of a group with this absolute maximum.
+__device__ __forceinline__ uint16_t q6_scale_bits(float amax) {
   const _Float16 hs = static_cast<_Float16>(__fdiv_rn(amax, 31.f));  // round to nearest even
   uint16_t sbits = __builtin_bit_cast(uint16_t, hs);
   if ((sbits & 0x7fffu) == 0x7c00u) sbits = (sbits & 0x8000u) | 0x7bffu;  // saturate +inf
-  const float sc = half_bits_to_f32(sbits);
-  uint32_t w = 0;
-#pragma unroll
-  for (int e = 0; e < kGroup; ++e) {
-    int c = 0;
-    if (sc != 0.f) {
-      const float r = rintf(__fdiv_rn(x[e], sc));
-      c = static_cast<int>(fminf(fmaxf(r, -31.f), 31.f));
-    }
-    w |= (static_cast<uint32_t>(c) & 63u) << (6 * (e & 3));
-    if ((e & 3) == 3) {
-      const int k = e >> 2;
-      codes24[3 * k + 0] = static_cast<uint8_t>(w);
-      codes24[3 * k + 1] = static_cast<uint8_t>(w >> 8);
-      codes24[3 * k + 2] = static_cast<uint8_t>(w >> 16);
-      w = 0;
-    }
-  }
   return sbits;
+}
+
+// Codes clamp(rint(x / sc), -31, 31) of one lane's 8 values, as floats.  The
+// quotient is formed as x * (1 / sc).  With sc a normal fp16 value below its
+// largest, |x / sc| <= 31 (1 + 2^-11): nothing clamps, and the product is
+// within 9e-6 of the rounded division, so one further than 2e-5 from every
+// half-way point rounds to the same integer.  The rest (a subnormal or
+// saturated scale, a NaN, a value near half-way: about one lane group in
+// 1,600 for Gaussian rows) takes the division and the clamp, which for every
+// value were two thirds of the instructions.
+__device__ __forceinline__ void q6_lane_codes(const float* x, float sc, float* c) {
+  const float inv = __builtin_amdgcn_rcpf(sc);
+  bool rest = !(sc >= 6.1035156e-5f && sc < 65504.f);
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const float q = x[e] * inv;
+    c[e] = rintf(q);
+    rest |= !(fabsf(q - c[e]) <= 0.5f - 2e-5f);
+  }
+  if (rest) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+      c[e] = sc == 0.f ? 0.f : fminf(fmaxf(rintf(__fdiv_rn(x[e], sc)), -31.f), 31.f);
+  }
+}
+
+// Four codes as the low 24 bits: sum (c_i + 32) 64^i is exact in fp32, and
+// flipping bit 5 of each field turns c + 32 into c's low six bits.
+__device__ __forceinline__ uint32_t q6_pack4(const float* c) {
+  const float w = fmaf(fmaf(fmaf(c[3], 64.f, c[2]), 64.f, c[1]), 64.f, c[0]);
+  return static_cast<uint32_t>(w + 8521760.f) ^ 0x820820u;   // 32 (1 + 64 + 64^2 + 64^3)
 }
 
 // 32 signed codes of one group from its 24 bytes (6 dwords, 4-byte aligned).
@@ -83,61 +93,167 @@ __device__ __forceinline__ void q6_codes(const uint8_t* p, float* c) {
   }
 }
 
-template <typename T>
-__global__ __launch_bounds__(kBlock) void q6_pack_kernel(int B, int Hkv, int N, const T* __restrict__ k,
-                                                         const int64_t* ks, const T* __restrict__ v,
-                                                         const int64_t* vs, uint8_t* __restrict__ cache,
-                                                         const int64_t* cs, const float* __restrict__ kprobe,
-                                                         int64_t ks0, int64_t ks1, int64_t ks2, int64_t vs0,
-                                                         int64_t vs1, int64_t vs2, int64_t cs0, int64_t cs1,
-                                                         int64_t cs2) {
-  (void)ks; (void)vs; (void)cs;
-  const int64_t idx = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
-  if (idx >= static_cast<int64_t>(B) * Hkv * N) return;
-  const int t = idx % N;
-  const int hk = (idx / N) % Hkv;
-  const int b = idx / (static_cast<int64_t>(N) * Hkv);
-  float kr[kHeadDim], vr[kHeadDim];
-  load_f32<T, kHeadDim>(k + b * ks0 + hk * ks1 + static_cast<int64_t>(t) * ks2, kr);
-  load_f32<T, kHeadDim>(v + b * vs0 + hk * vs1 + static_cast<int64_t>(t) * vs2, vr);
-  alignas(16) uint8_t slot[kSlot];
+// The broadcast of lane L of each quad.
+template <int L>
+__device__ __forceinline__ float quad_bcast(float x) {
+  return dpp_f<L * 0x55>(x);
+}
+
+// acc += x p and ss += x^2 over the eight dims held by lane L of the quad, in
+// dim order.  Each x is broadcast into the product with the lane's own probe;
+// the sum of squares runs on in every lane and lane L's is taken.
+template <int L>
+__device__ __forceinline__ void probe_chain(const float* x, const float* p, float& ss, float& acc) {
 #pragma unroll
-  for (int i = 0; i < kSlot; ++i) slot[i] = 0;
-  uint16_t sk0 = q6_quantize_group(kr, slot + kKCodes);
-  uint16_t sk1 = q6_quantize_group(kr + kGroup, slot + kKCodes + 24);
-  uint16_t sv0 = q6_quantize_group(vr, slot + kVCodes);
-  uint16_t sv1 = q6_quantize_group(vr + kGroup, slot + kVCodes + 24);
-  slot[kKScales + 0] = sk0 & 0xff; slot[kKScales + 1] = sk0 >> 8;
-  slot[kKScales + 2] = sk1 & 0xff; slot[kKScales + 3] = sk1 >> 8;
-  slot[kVScales + 0] = sv0 & 0xff; slot[kVScales + 1] = sv0 >> 8;
-  slot[kVScales + 2] = sv1 & 0xff; slot[kVScales + 3] = sv1 >> 8;
-  if (kprobe) {
-    // z from the dequantised K row, as the prefill/decode kernels see it.
-    float kq[kHeadDim];
-    q6_codes(slot + kKCodes, kq);
-    q6_codes(slot + kKCodes + 24, kq + kGroup);
-    const float s0 = half_bits_to_f32(sk0), s1 = half_bits_to_f32(sk1);
-    float ss = 0.f;
+  for (int e = 0; e < 8; ++e) acc = fmaf(quad_bcast<L>(x[e]), p[8 * L + e], acc);
 #pragma unroll
-    for (int d = 0; d < kHeadDim; ++d) {
-      kq[d] *= d < kGroup ? s0 : s1;
-      ss = fmaf(kq[d], kq[d], ss);
-    }
-    const float inv = rsqrtf(ss + 1e-6f * kHeadDim);
-    float z[4];
+  for (int e = 0; e < 8; ++e) ss = fmaf(x[e], x[e], ss);
+  ss = quad_bcast<L>(ss);
+}
+
+// One slot per row, four lanes to a row: lane l holds dims [8l, 8l + 8) of
+// each of the row's four groups (K0, K1, V0, V1), so a wave load covers 16
+// rows by 64 contiguous bytes, a group's maximum is two quad steps, and a
+// lane's eight codes are six whole bytes of the group's 24.  z is summed over
+// the 64 dims in order (lane r the plane r), each dim broadcast over the quad.
+// The 16 finished slots go through LDS and leave as whole 16-byte pieces of
+// consecutive slots.  Persistent waves keep their plane's probe in registers
+// and request the next 16 rows before they work on these.
+// At 327,680 bf16 rows (84 MB read, 42 MB written) 37 us, 3.4 TB/s, bound by
+// VALU issue (about 700 instructions a step, a 23 us floor) and then memory;
+// one thread per row, each reading and writing its own lines and dividing
+// every value, took 83 us.  Holding the kernel to 128 VGPRs for a fourth
+// workgroup per CU spills the probes: 57 us.
+template <typename T, bool PROBE>
+__global__ __launch_bounds__(kBlock) void q6_pack_kernel(unsigned Hkv, unsigned N, int64_t rows, const T* __restrict__ k,
+                                                         const T* __restrict__ v, uint8_t* __restrict__ cache,
+                                                         const float* __restrict__ kprobe, int64_t ks0, int64_t ks1,
+                                                         int64_t ks2, int64_t vs0, int64_t vs1, int64_t vs2,
+                                                         int64_t cs0, int64_t cs1, int64_t cs2) {
+  constexpr int kRows = kWave / 4;
+  constexpr int kPieces = sizeof(T) / 2;   // 16-byte pieces of eight values
+  __shared__ __align__(16) uint8_t s_slot[kBlock / kWave][kRows * kSlot];
+  const int lane = threadIdx.x % kWave, l = lane & 3, i = lane >> 2;
+  uint8_t* sw = s_slot[threadIdx.x / kWave];
+  uint8_t* mine = sw + i * kSlot;
+  float p[PROBE ? kHeadDim : 1];
+  if constexpr (PROBE) {
 #pragma unroll
-    for (int r = 0; r < kPlanes; ++r) {
-      float acc = 0.f;
-      for (int d = 0; d < kHeadDim; ++d) acc = fmaf(kq[d], kprobe[r * kHeadDim + d], acc);
-      z[r] = acc * inv;
-    }
-    float* zp = reinterpret_cast<float*>(slot + kZ);
-    zp[0] = z[0]; zp[1] = z[1]; zp[2] = z[2]; zp[3] = z[3];
+    for (int d = 0; d < kHeadDim; ++d) p[d] = kprobe[l * kHeadDim + d];
   }
-  uint4* dst = reinterpret_cast<uint4*>(cache + b * cs0 + hk * cs1 + static_cast<int64_t>(t) * cs2);
-  const uint4* src = reinterpret_cast<const uint4*>(slot);
+  const int64_t stride = static_cast<int64_t>(gridDim.x) * (kBlock / kWave) * kRows;
+  int64_t row0 = (static_cast<int64_t>(blockIdx.x) * (kBlock / kWave) + uniform(threadIdx.x / kWave)) * kRows;
+  if (row0 >= rows) return;
+  // (b, kv head, t) of row0 and of a step's advance: divided once, then carried (a 64-bit division per step on the
+  // scalar unit took longer than the step's loads)
+  const int64_t head0 = row0 / N, headS = stride / N;
+  unsigned t0 = static_cast<unsigned>(row0 - head0 * N), h0 = static_cast<unsigned>(head0 % Hkv),
+           b0 = static_cast<unsigned>(head0 / Hkv);
+  const unsigned tS = static_cast<unsigned>(stride - headS * N), hS = static_cast<unsigned>(headS % Hkv),
+                 bS = static_cast<unsigned>(headS / Hkv);
+  uint4 raw[4][kPieces];
+  uint8_t* out;
+  // rows past the end read the last one and store nothing
+  auto fetch = [&](int64_t left) {
+    const unsigned last = static_cast<unsigned>(left < kRows ? left : kRows) - 1;
+    const unsigned tt = t0 + (static_cast<unsigned>(i) < last ? i : last);
+    const unsigned up = tt / N, t = tt - up * N;
+    const unsigned hh = h0 + up, ub = hh / Hkv, hk = hh - ub * Hkv, b = b0 + ub;
+    const uint4* kp = reinterpret_cast<const uint4*>(k + b * ks0 + hk * ks1 + t * ks2);
+    const uint4* vp = reinterpret_cast<const uint4*>(v + b * vs0 + hk * vs1 + t * vs2);
+    out = cache + b * cs0 + hk * cs1 + t * cs2;
 #pragma unroll
-  for (int i = 0; i < kSlot / 16; ++i) dst[i] = src[i];
+    for (int g = 0; g < 2; ++g)
+#pragma unroll
+      for (int w = 0; w < kPieces; ++w) {
+        raw[g][w] = kp[(4 * g + l) * kPieces + w];
+        raw[2 + g][w] = vp[(4 * g + l) * kPieces + w];
+      }
+  };
+  fetch(rows - row0);
+  for (; row0 < rows; row0 += stride) {
+    float x[4][8];
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      if constexpr (kPieces == 1) {
+        const uint32_t w[4] = {raw[g][0].x, raw[g][0].y, raw[g][0].z, raw[g][0].w};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) { x[g][2 * e] = bf16_lo(w[e]); x[g][2 * e + 1] = bf16_hi(w[e]); }
+      } else {
+#pragma unroll
+        for (int w = 0; w < kPieces; ++w) {
+          x[g][4 * w] = __uint_as_float(raw[g][w].x); x[g][4 * w + 1] = __uint_as_float(raw[g][w].y);
+          x[g][4 * w + 2] = __uint_as_float(raw[g][w].z); x[g][4 * w + 3] = __uint_as_float(raw[g][w].w);
+        }
+      }
+    }
+    uint8_t* const dst_row = out;
+    if (row0 + stride < rows) {
+      t0 += tS;
+      h0 += hS + (t0 >= N);
+      t0 -= t0 >= N ? N : 0;
+      b0 += bS + (h0 >= Hkv);
+      h0 -= h0 >= Hkv ? Hkv : 0;
+      fetch(rows - row0 - stride);
+    }
+    float amax[4];
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      amax[g] = 0.f;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) amax[g] = fmaxf(amax[g], fabsf(x[g][e]));
+      amax[g] = fmaxf(amax[g], dpp_f<0xB1>(amax[g]));
+      amax[g] = fmaxf(amax[g], dpp_f<0x4E>(amax[g]));
+    }
+    // lane g forms group g's scale
+    const uint32_t own = q6_scale_bits(pick4(l, amax[0], amax[1], amax[2], amax[3]));
+    const float ownf = __uint_as_float(own);
+    const uint32_t sbits[4] = {__float_as_uint(quad_bcast<0>(ownf)), __float_as_uint(quad_bcast<1>(ownf)),
+                               __float_as_uint(quad_bcast<2>(ownf)), __float_as_uint(quad_bcast<3>(ownf))};
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const float sc = half_bits_to_f32(static_cast<uint16_t>(sbits[g]));
+      float c[8];
+      q6_lane_codes(x[g], sc, c);
+      const uint32_t w0 = q6_pack4(c), w1 = q6_pack4(c + 4);
+      uint16_t* dst = reinterpret_cast<uint16_t*>(mine + (g < 2 ? kKCodes : kVCodes) + 24 * (g & 1) + 6 * l);
+      dst[0] = static_cast<uint16_t>(w0);
+      dst[1] = static_cast<uint16_t>((w0 >> 16) | (w1 << 8));
+      dst[2] = static_cast<uint16_t>(w1 >> 8);
+      if (PROBE && g < 2) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[g][e] = c[e] * sc;   // the dequantised K row, exact
+      }
+    }
+    const uint32_t scales = l == 0 ? sbits[0] | (sbits[1] << 16) : sbits[2] | (sbits[3] << 16);
+    if (l < 2) *reinterpret_cast<uint32_t*>(mine + (l == 0 ? kKScales : kVScales)) = scales;
+    else *reinterpret_cast<uint32_t*>(mine + kZ + 16 + 4 * (l - 2)) = 0;
+    float z = 0.f;
+    if constexpr (PROBE) {
+      // z from the dequantised K row, as the prefill and decode kernels see it
+      float ss = 0.f, acc = 0.f;
+      probe_chain<0>(x[0], p, ss, acc);
+      probe_chain<1>(x[0], p, ss, acc);
+      probe_chain<2>(x[0], p, ss, acc);
+      probe_chain<3>(x[0], p, ss, acc);
+      probe_chain<0>(x[1], p + kGroup, ss, acc);
+      probe_chain<1>(x[1], p + kGroup, ss, acc);
+      probe_chain<2>(x[1], p + kGroup, ss, acc);
+      probe_chain<3>(x[1], p + kGroup, ss, acc);
+      z = acc * rsqrtf(ss + 1e-6f * kHeadDim);
+    }
+    *reinterpret_cast<float*>(mine + kZ + 4 * l) = z;
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    const uint4* src = reinterpret_cast<const uint4*>(mine);
+    const uint4 o0 = src[l], o1 = src[4 + l];
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    __builtin_amdgcn_wave_barrier();   // the next 16 rows overwrite these slots
+    if (row0 + i < rows) {
+      reinterpret_cast<uint4*>(dst_row)[l] = o0;
+      reinterpret_cast<uint4*>(dst_row)[4 + l] = o1;
+    }
+  }
 }
 
 __global__ __launch_bounds__(kBlock) void q6_unpack_kernel(int B, int Hkv, int N, const uint8_t* __restrict__ cache,
@@ -1339,15 +1455,22 @@ hipError_t launch_q6_pack(int B, int Hkv, int N, int dtype, const void* k, const
                           const int64_t* vs, uint8_t* cache, const int64_t* cs, const float* kprobe,
                           hipStream_t stream) {
   const int64_t rows = static_cast<int64_t>(B) * Hkv * N;
-  const int blocks = static_cast<int>((rows + kBlock - 1) / kBlock);
-  if (dtype == DWARF_BF16)
-    hipLaunchKernelGGL(q6_pack_kernel<bf16>, dim3(blocks), dim3(kBlock), 0, stream, B, Hkv, N,
-                       static_cast<const bf16*>(k), nullptr, static_cast<const bf16*>(v), nullptr, cache, nullptr,
-                       kprobe, ks[0], ks[1], ks[2], vs[0], vs[1], vs[2], cs[0], cs[1], cs[2]);
-  else
-    hipLaunchKernelGGL(q6_pack_kernel<float>, dim3(blocks), dim3(kBlock), 0, stream, B, Hkv, N,
-                       static_cast<const float*>(k), nullptr, static_cast<const float*>(v), nullptr, cache, nullptr,
-                       kprobe, ks[0], ks[1], ks[2], vs[0], vs[1], vs[2], cs[0], cs[1], cs[2]);
+  // 64 rows to a workgroup and step; from 768 workgroups on, persistent: three per CU are resident at once (37 us at
+  // 327,680 rows; 38 with 1,024 workgroups, 47 with one per step, which loads the probes again each time)
+  const int64_t want = (rows + kBlock / 4 - 1) / (kBlock / 4);
+  const int blocks = static_cast<int>(want < 768 ? want : 768);
+#define DWARF_Q6_PACK(T, P)                                                                                      \
+  hipLaunchKernelGGL((q6_pack_kernel<T, P>), dim3(blocks), dim3(kBlock), 0, stream, static_cast<unsigned>(Hkv),  \
+                     static_cast<unsigned>(N), rows, static_cast<const T*>(k), static_cast<const T*>(v), cache,  \
+                     kprobe, ks[0], ks[1], ks[2], vs[0], vs[1], vs[2], cs[0], cs[1], cs[2])
+  if (dtype == DWARF_BF16) {
+    if (kprobe) DWARF_Q6_PACK(bf16, true);
+    else DWARF_Q6_PACK(bf16, false);
+  } else {
+    if (kprobe) DWARF_Q6_PACK(float, true);
+    else DWARF_Q6_PACK(float, false);
+  }
+#undef DWARF_Q6_PACK
   return hipGetLastError();
 }
 

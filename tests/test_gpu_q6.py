@@ -44,6 +44,38 @@ def test_pack_matches_cpu_codec_bit_exact(pkg, device, dtype):
     assert np.allclose(z, rz, rtol=1e-5, atol=1e-6)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("B,Hkv,N,probes", [(1, 1, 1, True), (2, 3, 5, True), (1, 2, 16, False), (3, 1, 17, True),
+                                            (1, 7, 9400, True)])
+def test_pack_row_remainders(pkg, device, B, Hkv, N, probes, dtype):
+    """The pack's 16-row steps: one row, heads shorter than a step, a last step of one row, and enough rows that a
+    persistent wave takes a second step; K and V as head-interleaved views.  Rows at k + 1/2 of their scale take the
+    codec's exact division, others the reciprocal: both must give the CPU codec's bytes.  z: 64 fp32 products and
+    sums of unit-bounded terms, within 64 ulps of 1 (8e-6)."""
+    g = torch.Generator().manual_seed(N)
+    k = torch.randn(B, N, Hkv, 64, generator=g)
+    k[:, 0, :, :32] = (torch.arange(32) - 15.5)[None, None]     # scale 0.5: x / s = odd integers; and halves below
+    k[:, 0, :, 32:] = torch.cat((torch.tensor([31.0]), torch.arange(31) - 14.5))[None, None]   # scale 1: half-way codes
+    v = 2.0 * torch.randn(B, N, Hkv, 64, generator=g)
+    v[0, N // 2, 0, 3], v[0, N // 2, 0, 40] = float("nan"), float("inf")
+    k, v = k.to(dtype).transpose(1, 2), v.to(dtype).transpose(1, 2)
+    kpn = torch.nn.functional.normalize(torch.randn(4, 64, generator=g), dim=-1)
+    cache = pkg.q6.pack_kv(k.to(device), v.to(device), kpn.to(device) if probes else None).cpu().numpy()
+    bad = ~np.isfinite(v.float().numpy())
+    ref = q6_ref.pack_slots(k.float().numpy(), np.where(bad, 0.0, v.float().numpy()).astype(np.float32), None)
+    keep = ~bad.any(-1)                                          # the codec states no code for a group with NaN or inf
+    assert np.array_equal(cache[..., :52], ref[..., :52])
+    assert np.array_equal(cache[keep][..., :104], ref[keep][..., :104])
+    assert not cache[..., 120:].any()
+    z = np.ascontiguousarray(cache[..., 104:120]).view(np.float32)
+    if not probes:
+        assert not z.any()
+        return
+    rk, _, _ = q6_ref.unpack_slots(cache)
+    rz = features(torch.from_numpy(rk).double(), kpn).numpy()
+    assert np.abs(z - rz).max() < 8e-6
+
+
 def _oracle_on_cache(x, cache_np, offsets, js, shift, qp, kp, qs, return_lse=False, round_se=True):
     kd, vd, _ = q6_ref.unpack_slots(cache_np)
     inp = dict(x)
