@@ -280,6 +280,34 @@ class PacketBwdArgs(ctypes.Structure):
     ]
 
 
+# ---- include/dwarf_block.h ----
+BLOCK_SYMBOLS = ("dwarf_head_gate_fwd", "dwarf_head_gate_bwd_workspace_bytes", "dwarf_head_gate_bwd")
+
+
+class HeadGateFwdArgs(ctypes.Structure):
+    _fields_ = [
+        ("B", c_int32), ("H", c_int32), ("N", c_int32),
+        ("out", c_void_p), ("out_stride", _i64(4)),
+        ("gain", c_void_p),
+        ("gate", c_void_p), ("gate_stride", _i64(3)),
+        ("gated", c_void_p), ("gated_stride", _i64(3)),
+    ]
+
+
+class HeadGateBwdArgs(ctypes.Structure):
+    _fields_ = [
+        ("fwd", HeadGateFwdArgs),
+        ("dgated", c_void_p), ("dgated_stride", _i64(3)),
+        ("dout", c_void_p), ("dout_stride", _i64(4)),
+        ("dgate", c_void_p), ("dgate_stride", _i64(3)),
+        ("dgain", c_void_p),
+        ("lse", c_void_p), ("lse_stride", _i64(3)),
+        ("query_start", c_int32),
+        ("delta_pairs", c_void_p),
+        ("workspace", c_void_p), ("workspace_bytes", c_size_t),
+    ]
+
+
 class NativeLibraryError(RuntimeError):
     """The HIP library is missing, stale or failed a call."""
 
@@ -368,6 +396,12 @@ def load() -> ctypes.CDLL:
     lib.dwarf_packet_bwd_workspace_bytes.argtypes = [POINTER(PacketBwdArgs)]
     lib.dwarf_packet_bwd.restype = c_int
     lib.dwarf_packet_bwd.argtypes = [POINTER(PacketBwdArgs), c_void_p]
+    lib.dwarf_head_gate_fwd.restype = c_int
+    lib.dwarf_head_gate_fwd.argtypes = [POINTER(HeadGateFwdArgs), c_void_p]
+    lib.dwarf_head_gate_bwd_workspace_bytes.restype = c_size_t
+    lib.dwarf_head_gate_bwd_workspace_bytes.argtypes = [POINTER(HeadGateBwdArgs)]
+    lib.dwarf_head_gate_bwd.restype = c_int
+    lib.dwarf_head_gate_bwd.argtypes = [POINTER(HeadGateBwdArgs), c_void_p]
     version = lib.dwarf_abi_version()
     if version != ABI_VERSION:
         raise NativeLibraryError(f"{LIB_NAME} ABI {version} does not match the binding's ABI {ABI_VERSION}")

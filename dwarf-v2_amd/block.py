@@ -20,31 +20,40 @@ centered_scale_embed, phase_base, phase_gain, j_val, j_small, j_large,
 offsets_dev, the five sparse-plan buffers, k_group_size, grouped_mode_id,
 verify_mode, max_group_spread_observed, plane_shift, backend,
 online_softmax, if_gain, out_proj, dropout.
+
+Under bf16 autocast, without kv_inject and without support cropping (the
+trainer's blocks), everything between the two projections is one autograd
+Function on the fused projection [B, N, 4D] (``_DSQGBlockFn``): the attention
+reads q, k and v as views of it, the per-head gain and the content gate are
+one launch after it (csrc/block.hip), and the backward writes dq, dk, dv and
+the gate's gradient straight into one [B, N, 4D] gradient.  Each product is
+rounded where the unfused expression rounds it.
 """
 
 from __future__ import annotations
 
+import ctypes
+
 import torch
 import torch.nn.functional as F
 
-from .dsqg import dsqg_attention_with_probes
+from . import _lib
+from .dsqg import (HEAD_DIM, _check_call, _planes, _rows_ok, _stream, dsqg_attention_with_probes, dsqg_backward,
+                   dsqg_forward, normalize_inputs, schedule_for)
 from .npci import npci_rotate
+from .probe import probe_forward
 
 NPCI_THETA_MAX = 0.25   # bound of the NPCI rotation angle, theta = 0.25 tanh(raw) (dsqg:71, 3216, 3222)
 
 
-def _projections(block, x: torch.Tensor, query_start: int, key_end: int):
-    """q, k, v and the content gate, each [B, N, D].
+def _cropped_projections(block, x: torch.Tensor, query_start: int, key_end: int):
+    """q, k, v and the content gate, each [B, N, D], under support cropping (dsqg:3158-3187).
 
-    With support cropping (dsqg:3158-3187) only the rows that can take part
-    are projected: q and the gate for rows >= query_start (no offset reaches
-    an earlier query), k and v for rows < key_end (no query reaches a later
-    source); the other rows are zero.  Otherwise one fused projection.
+    Only the rows that can take part are projected: q and the gate for rows
+    >= query_start (no offset reaches an earlier query), k and v for rows
+    < key_end (no query reaches a later source); the other rows are zero.
     """
     D = x.shape[-1]
-    crop = block.support_crop_projections and query_start >= block.support_crop_min_offset
-    if not crop:
-        return block.qkvg_proj(x).split(D, dim=-1)
     w, b = block.qkvg_proj.weight, block.qkvg_proj.bias
     q, k, v, gate = (x.new_zeros(x.shape) for _ in range(4))
     tail, head = x[:, query_start:], x[:, :key_end]
@@ -53,6 +62,157 @@ def _projections(block, x: torch.Tensor, query_start: int, key_end: int):
     kv = F.linear(head, w[D:3 * D], b[D:3 * D])
     k[:, :key_end], v[:, :key_end] = kv[..., :D], kv[..., D:]
     return q, k, v, gate
+
+
+def _heads(t: torch.Tensor, heads: int) -> torch.Tensor:
+    """[B, N, H*64] -> [B, H, N, 64] view."""
+    B, N, D = t.shape
+    return t.reshape(B, N, heads, D // heads).permute(0, 2, 1, 3)
+
+
+def _fill_gate(a: _lib.HeadGateFwdArgs, out, gain, gate) -> None:
+    a.B, a.H, a.N = out.shape[:3]
+    a.out, a.out_stride = out.data_ptr(), _lib.i64_array(out.stride())
+    a.gain = gain.data_ptr()
+    a.gate, a.gate_stride = gate.data_ptr(), _lib.i64_array(gate.stride())
+
+
+def head_gate_forward(out: torch.Tensor, gain: torch.Tensor, gate: torch.Tensor) -> torch.Tensor:
+    """Raw launch: bf16((out * gain[h]) * bf16(sigmoid(gate))) as [B,N,H*64]; out bf16 [B,H,N,64], gain fp32
+    [H], gate bf16 [B,N,H*64]."""
+    lib = _lib.load()
+    B, H, N, hd = out.shape
+    gated = torch.empty((B, N, H * hd), device=out.device, dtype=out.dtype)
+    a = _lib.HeadGateFwdArgs()
+    _fill_gate(a, out, gain, gate)
+    a.gated, a.gated_stride = gated.data_ptr(), _lib.i64_array(gated.stride())
+    _lib.check(lib.dwarf_head_gate_fwd(ctypes.byref(a), _stream(out.device)), "dwarf_head_gate_fwd")
+    return gated
+
+
+def head_gate_backward(dgated, out, gain, gate, dgate, *, lse=None, query_start=0, pairs=0):
+    """Raw launch: (dout like out, dgain fp32 [H]); the gate's gradient goes into ``dgate``.  pairs: address
+    of the [B,H,N] (delta, lse) pairs to write as well, 0 for none."""
+    lib = _lib.load()
+    dout = torch.empty_like(out)
+    dgain = torch.empty(gain.shape, device=out.device, dtype=torch.float32)
+    a = _lib.HeadGateBwdArgs()
+    _fill_gate(a.fwd, out, gain, gate)
+    a.dgated, a.dgated_stride = dgated.data_ptr(), _lib.i64_array(dgated.stride())
+    a.dout, a.dout_stride = dout.data_ptr(), _lib.i64_array(dout.stride())
+    a.dgate, a.dgate_stride = dgate.data_ptr(), _lib.i64_array(dgate.stride())
+    a.dgain = dgain.data_ptr()
+    if pairs:
+        a.delta_pairs, a.query_start = pairs, int(query_start)
+        a.lse, a.lse_stride = lse.data_ptr(), _lib.i64_array(lse.stride())
+    ws = torch.empty(max(int(lib.dwarf_head_gate_bwd_workspace_bytes(ctypes.byref(a))), 16), device=out.device,
+                     dtype=torch.uint8)
+    a.workspace, a.workspace_bytes = ws.data_ptr(), ws.numel()
+    _lib.check(lib.dwarf_head_gate_bwd(ctypes.byref(a), _stream(out.device)), "dwarf_head_gate_bwd")
+    return dout, dgain
+
+
+def block_forward(qkvg, pos_bias, scale_embed, phase_base, phase_gain, query_probes, key_probes, gain, offsets, heads,
+                  j_small, j_large, plane_shift, query_start, schedule):
+    """Raw launches from the fused projection [B,N,4D] (bf16, contiguous) to the gated heads [B,N,D]: returns
+    (gated, out [B,N,H,64], lse, y, z)."""
+    qkvg = qkvg if qkvg.is_contiguous() and _rows_ok(qkvg) else qkvg.clone(memory_format=torch.contiguous_format)
+    B, N, D4 = qkvg.shape
+    q, k, v, gate = qkvg.split(D4 // 4, dim=-1)
+    q, k, v = (_heads(t, heads) for t in (q, k, v))
+    z = probe_forward(k, key_probes, 0, N)
+    t = normalize_inputs(q, k, v, pos_bias, scale_embed, phase_base, phase_gain, None, z, offsets, j_small + j_large)
+    out = torch.empty((B, N, heads, HEAD_DIM), device=qkvg.device, dtype=qkvg.dtype)
+    _, lse, y = dsqg_forward(*t, j_small, j_large, plane_shift, query_start, schedule=schedule,
+                             query_probes=_planes(query_probes.float()), out=out.permute(0, 2, 1, 3))
+    gated = head_gate_forward(out.permute(0, 2, 1, 3), gain.float().contiguous(), gate)
+    return gated, out, lse, y, z
+
+
+def block_backward(dgated, qkvg, pos_bias, scale_embed, phase_base, phase_gain, query_probes, key_probes, gain, offsets,
+                   out, lse, y, z, heads, j_small, j_large, plane_shift, query_start, schedule):
+    """Raw launches: (dqkvg [B,N,4D], dpos_bias, dscale_embed, dphase_base, dphase_gain, dgain)."""
+    qkvg = qkvg if qkvg.is_contiguous() and _rows_ok(qkvg) else qkvg.clone(memory_format=torch.contiguous_format)
+    D = qkvg.shape[-1] // 4
+    dgated = dgated.to(qkvg.dtype)
+    dgated = dgated if _rows_ok(dgated) else dgated.clone(memory_format=torch.contiguous_format)
+    dqkvg = torch.empty_like(qkvg)
+    q, k, v, gate = qkvg.split(D, dim=-1)
+    dq, dk, dv, dgate = dqkvg.split(D, dim=-1)
+    q, k, v, dq, dk, dv = (_heads(t, heads) for t in (q, k, v, dq, dk, dv))
+    o = out.contiguous().permute(0, 2, 1, 3)
+    lse = lse.contiguous()
+    t = normalize_inputs(q, k, v, pos_bias, scale_embed, phase_base, phase_gain, y, z, offsets, j_small + j_large)
+    gain = gain.float().contiguous()
+    dgain = None
+
+    def gate_launch(pairs):
+        nonlocal dgain
+        dout, dgain = head_gate_backward(dgated, o, gain, gate, dgate, lse=lse, query_start=query_start, pairs=pairs)
+        return dout
+
+    g = dsqg_backward(gate_launch, *t, o, lse, j_small, j_large, plane_shift, query_start, schedule=schedule,
+                      query_probes=_planes(query_probes.float()), key_probes=_planes(key_probes.float()),
+                      into=(dq, dk, dv))
+    return (dqkvg, *g[3:7], dgain)
+
+
+class _DSQGBlockFn(torch.autograd.Function):
+    """The block between its projections as one node: gated heads from the fused projection, over the custom
+    ops ``torch.ops.dwarf.dsqg_block_fwd`` / ``dsqg_block_bwd`` (registered in ``ops.py``).  Probes: normalised
+    fp32 [4,64], without gradient."""
+
+    @staticmethod
+    def forward(ctx, qkvg, pos_bias, scale_embed, phase_base, phase_gain, gain, query_probes, key_probes, offsets_dev,
+                heads, j_small, j_large, plane_shift, query_start, schedule):
+        ctx.args = (int(heads), int(j_small), int(j_large), int(plane_shift), int(query_start), int(schedule))
+        gated, out, lse, y, z = torch.ops.dwarf.dsqg_block_fwd(qkvg, pos_bias, scale_embed, phase_base, phase_gain,
+                                                               query_probes, key_probes, gain, offsets_dev, *ctx.args)
+        ctx.save_for_backward(qkvg, pos_bias, scale_embed, phase_base, phase_gain, gain, query_probes, key_probes,
+                              offsets_dev, out, lse, y, z)
+        return gated
+
+    @staticmethod
+    def backward(ctx, dgated):
+        qkvg, pb, se, pbase, pgain, gain, qp, kp, offsets, out, lse, y, z = ctx.saved_tensors
+        g = torch.ops.dwarf.dsqg_block_bwd(dgated, qkvg, pb, se, pbase, pgain, qp, kp, gain, offsets, out, lse, y, z,
+                                           *ctx.args)
+        dqkvg, dpb, dse, dpbase, dpgain, dgain = g
+        return (dqkvg, dpb, dse, dpbase, dpgain, dgain.reshape(gain.shape)) + (None,) * 9
+
+
+def _plain_linear(m) -> bool:
+    """An nn.Linear nothing hooks into: it takes the bf16 product where autocast would have cast an fp32 one."""
+    return (type(m) is torch.nn.Linear and not m._forward_pre_hooks and not m._forward_hooks
+            and not m._backward_hooks and not m._backward_pre_hooks)
+
+
+def _one_node(block, proj: torch.Tensor) -> bool:
+    """Whether the block between its projections runs as ``_DSQGBlockFn``: bf16 autocast (so that the output
+    projection reads bf16 either way), frozen phase probes, the fp32 gain of the module."""
+    if not (proj.is_cuda and proj.dtype == torch.bfloat16 and torch.is_autocast_enabled("cuda")
+            and torch.get_autocast_dtype("cuda") == torch.bfloat16):
+        return False
+    if torch.is_grad_enabled() and (block.query_probes.requires_grad or block.key_probes.requires_grad):
+        return False
+    return (block.head_dim == HEAD_DIM and proj.shape[-1] == 4 * block.num_heads * HEAD_DIM
+            and block.if_gain.dtype == torch.float32 and block.if_gain.numel() == block.num_heads
+            and str(block.backend).lower() in ("auto", "triton", "hip") and _plain_linear(block.out_proj))
+
+
+def _gated_heads(block, proj: torch.Tensor, query_start: int) -> torch.Tensor:
+    H = block.num_heads
+    q, k, v, _ = proj.split(proj.shape[-1] // 4, dim=-1)
+    q, k, v = (_heads(t, H) for t in (q, k, v))
+    _check_call(q, k, v, None, None, block.j_val, block.j_small, block.j_large, block.offsets_dev, block.grouped_mode_id)
+    qp = F.normalize(block.query_probes.detach().float(), dim=-1).to(proj.device)
+    kp = F.normalize(block.key_probes.detach().float(), dim=-1).to(proj.device)
+    phase_gate = torch.sigmoid(block.phase_gate)[:, None, None]
+    return _DSQGBlockFn.apply(
+        proj, block.pos_bias.float(), block.centered_scale_embed.float(), (block.phase_base * phase_gate).float(),
+        (block.phase_gain * phase_gate).float(), block.if_gain.reshape(-1), qp, kp, block.offsets_dev, H,
+        int(block.j_small), int(block.j_large), int(block.plane_shift), max(0, min(int(query_start), proj.shape[1])),
+        schedule_for(block.grouped_mode_id, bool(block.online_softmax)))
 
 
 def _inject(block, k: torch.Tensor, v: torch.Tensor, kv_inject, key_end: int):
@@ -89,7 +249,13 @@ def dsqg_block_forward(block, x: torch.Tensor, kv_inject=None) -> torch.Tensor:
     if query_start >= N:
         return torch.zeros_like(x)
     key_end = max(0, N - query_start)
-    q, k, v, gate = _projections(block, x, query_start, key_end)
+    if block.support_crop_projections and query_start >= block.support_crop_min_offset:
+        q, k, v, gate = _cropped_projections(block, x, query_start, key_end)
+    else:
+        proj = block.qkvg_proj(x)
+        if kv_inject is None and _one_node(block, proj):
+            return block.dropout(block.out_proj(_gated_heads(block, proj, query_start)))
+        q, k, v, gate = proj.split(D, dim=-1)
     # [B, N, H*hd] -> [B, H, N, hd] views over the projection rows
     q, k, v = (t.reshape(B, N, H, hd).permute(0, 2, 1, 3) for t in (q, k, v))
     if kv_inject is not None:

@@ -8,6 +8,7 @@
 #include <cstdio>
 
 #include "dsqg_internal.h"
+#include "dwarf_block.h"
 #include "dwarf_dsqg.h"
 
 namespace dwarf {
@@ -43,6 +44,9 @@ hipError_t launch_interference_packet_fwd(const dwarf_packet_fwd_args& a, hipStr
 hipError_t launch_interference_packet_bwd(const dwarf_packet_bwd_args& a, hipStream_t stream);
 hipError_t launch_phase_probe_fwd(const dwarf_phase_probe_fwd_args& a, hipStream_t stream);
 hipError_t launch_phase_probe_bwd(const dwarf_phase_probe_bwd_args& a, hipStream_t stream);
+size_t head_gate_bwd_workspace(const dwarf_head_gate_bwd_args& a);
+hipError_t launch_head_gate_fwd(const dwarf_head_gate_fwd_args& a, hipStream_t stream);
+hipError_t launch_head_gate_bwd(const dwarf_head_gate_bwd_args& a, hipStream_t stream);
 }  // namespace dwarf
 
 namespace {
@@ -719,6 +723,52 @@ int dwarf_dsqg_q6_decode_noalloc(const dwarf_dsqg_q6_decode_args* args, dwarf_st
   if (e != hipSuccess) return hip_status(e, "dwarf_dsqg_q6_decode_noalloc (device array address)");
   return hip_status(dwarf::launch_q6_decode(a, table, reinterpret_cast<hipStream_t>(stream)),
                     "dwarf_dsqg_q6_decode_noalloc");
+}
+
+// ---- the DSQG block's gain and gate -----------------------------------------
+static int check_gate(const dwarf_head_gate_fwd_args& a) {
+  if (a.B < 0 || a.H <= 0 || a.N < 0) return fail(DWARF_ERR_INVALID_ARGUMENT, "bad sizes B=%d H=%d N=%d", a.B, a.H, a.N);
+  // the kernels number (b, n, h) with 32 bits, one grid stride of slack above
+  if (static_cast<int64_t>(a.B) * a.N * a.H >= (int64_t(1) << 31))
+    return fail(DWARF_ERR_UNSUPPORTED, "B x N x H must stay below 2^31");
+  if (a.B == 0 || a.N == 0) return DWARF_OK;
+  int rc;
+  if ((rc = check_rows("out", a.out, a.out_stride, 3, DWARF_BF16))) return rc;
+  if ((rc = check_rows("gate", a.gate, a.gate_stride, 2, DWARF_BF16))) return rc;
+  if (!a.gain) return fail(DWARF_ERR_INVALID_ARGUMENT, "gain is NULL");
+  return DWARF_OK;
+}
+
+int dwarf_head_gate_fwd(const dwarf_head_gate_fwd_args* args, dwarf_stream_t stream) {
+  if (!args) return fail(DWARF_ERR_INVALID_ARGUMENT, "args is NULL");
+  int rc = check_gate(*args);
+  if (rc) return rc;
+  if (args->B == 0 || args->N == 0) return ok();
+  if ((rc = check_rows("gated", args->gated, args->gated_stride, 2, DWARF_BF16))) return rc;
+  return hip_status(dwarf::launch_head_gate_fwd(*args, reinterpret_cast<hipStream_t>(stream)), "dwarf_head_gate_fwd");
+}
+
+size_t dwarf_head_gate_bwd_workspace_bytes(const dwarf_head_gate_bwd_args* a) {
+  return a && a->fwd.H > 0 ? dwarf::head_gate_bwd_workspace(*a) : 0;
+}
+
+int dwarf_head_gate_bwd(const dwarf_head_gate_bwd_args* args, dwarf_stream_t stream) {
+  if (!args) return fail(DWARF_ERR_INVALID_ARGUMENT, "args is NULL");
+  const dwarf_head_gate_bwd_args& a = *args;
+  int rc = check_gate(a.fwd);
+  if (rc) return rc;
+  if (!a.dgain) return fail(DWARF_ERR_INVALID_ARGUMENT, "dgain is NULL");
+  if (a.fwd.B == 0 || a.fwd.N == 0)
+    return zero_floats(a.dgain, a.fwd.H, reinterpret_cast<hipStream_t>(stream), "dwarf_head_gate_bwd");
+  if ((rc = check_rows("dgated", a.dgated, a.dgated_stride, 2, DWARF_BF16))) return rc;
+  if ((rc = check_rows("dout", a.dout, a.dout_stride, 3, DWARF_BF16))) return rc;
+  if ((rc = check_rows("dgate", a.dgate, a.dgate_stride, 2, DWARF_BF16))) return rc;
+  if (a.delta_pairs && (!a.lse || (reinterpret_cast<uintptr_t>(a.delta_pairs) & 7u)))
+    return fail(DWARF_ERR_INVALID_ARGUMENT, "delta_pairs needs lse and 8-byte alignment");
+  const size_t need = dwarf::head_gate_bwd_workspace(a);
+  if (!a.workspace || a.workspace_bytes < need || !aligned16(a.workspace))
+    return fail(DWARF_ERR_WORKSPACE, "workspace needs %zu bytes, 16-byte aligned, got %zu", need, a.workspace_bytes);
+  return hip_status(dwarf::launch_head_gate_bwd(a, reinterpret_cast<hipStream_t>(stream)), "dwarf_head_gate_bwd");
 }
 
 }  // extern "C"

@@ -125,8 +125,10 @@ def normalize_inputs(q, k, v, pos_bias, scale_embed, phase_base, phase_gain, y_p
 
 def dsqg_forward(q, k, v, pos_bias, scale_embed, phase_base, phase_gain, y_pre, z_pre, offsets_dev,
                  j_small, j_large, plane_shift=0, query_start=0, *, events=None, schedule=None,
-                 query_probes=None):
+                 query_probes=None, out=None):
     """Raw forward launch: returns (out, lse).  q/k/v share one dtype (bf16 or fp32).
+
+    ``out``: where to write the output, [B,H,N,64] of q's dtype in any strides with 16-byte rows.
 
     ``events``: optional (start, end) torch.cuda.Event pair recorded around the
     launch on the current stream.  ``schedule``: DWARF_SCHED_* flags (None: the
@@ -137,7 +139,8 @@ def dsqg_forward(q, k, v, pos_bias, scale_embed, phase_base, phase_gain, y_pre, 
     """
     lib = _lib.load()
     B, H, N, _ = q.shape
-    out = torch.empty((B, H, N, q.shape[3]), device=q.device, dtype=q.dtype)
+    if out is None:
+        out = torch.empty((B, H, N, q.shape[3]), device=q.device, dtype=q.dtype)
     lse = torch.empty((B, H, N), device=q.device, dtype=torch.float32)
     args = _lib.DsqgFwdArgs()
     _fill_fwd(args, q, k, v, pos_bias, scale_embed, phase_base, phase_gain, y_pre, z_pre, offsets_dev,
@@ -168,8 +171,14 @@ def _side_stream(device: torch.device) -> torch.cuda.Stream:
 
 def dsqg_backward(dout, q, k, v, pos_bias, scale_embed, phase_base, phase_gain, y_pre, z_pre, offsets_dev,
                   out, lse, j_small, j_large, plane_shift=0, query_start=0, *, events=None, schedule=None,
-                  overlap=None, one_call=False, overlap_events=None, query_probes=None, key_probes=None):
+                  overlap=None, one_call=False, overlap_events=None, query_probes=None, key_probes=None,
+                  into=None):
     """Raw backward.  Returns (dq, dk, dv, dpb, dse, dpbase, dpgain, dy, dz).
+
+    ``into``: (dq, dk, dv) to write, each like its input in any strides with 16-byte rows.  ``dout`` may be a
+    function of the workspace's address (0 unless the stages overlap) that launches what forms dout on the
+    current stream and returns it; given the address it also writes the (delta, lse) pairs there, and the
+    delta stage's own launch is left out.
 
     bf16 (``overlap`` None or True, no ``events``): the delta stage and dK/dV
     run on a second stream beside dQ and the parameter gradients on the
@@ -191,10 +200,12 @@ def dsqg_backward(dout, q, k, v, pos_bias, scale_embed, phase_base, phase_gain, 
     """
     lib = _lib.load()
     dev = q.device
-    dout = _kernel_rows(dout.to(q.dtype))
-    dq = torch.empty(q.shape, device=dev, dtype=q.dtype)
-    dk = torch.empty(k.shape, device=dev, dtype=k.dtype)
-    dv = torch.empty(v.shape, device=dev, dtype=v.dtype)
+    if into is None:
+        dq = torch.empty(q.shape, device=dev, dtype=q.dtype)
+        dk = torch.empty(k.shape, device=dev, dtype=k.dtype)
+        dv = torch.empty(v.shape, device=dev, dtype=v.dtype)
+    else:
+        dq, dk, dv = into
     dpb = torch.empty(pos_bias.shape, device=dev, dtype=torch.float32)
     dse = torch.empty(scale_embed.shape, device=dev, dtype=torch.float32)
     # the reduction writes every [J_large, H, 4] entry; the [1, H, 4] tables of a
@@ -211,7 +222,6 @@ def dsqg_backward(dout, q, k, v, pos_bias, scale_embed, phase_base, phase_gain, 
     _fill_fwd(args.fwd, q, k, v, pos_bias, scale_embed, phase_base, phase_gain, y_pre, z_pre, offsets_dev,
               j_small, j_large, plane_shift, query_start, out, lse, se_round=q.dtype != torch.float32,
               schedule=schedule)
-    args.dout, args.dout_stride = dout.data_ptr(), _lib.i64_array(dout.stride())
     args.dq, args.dq_stride = dq.data_ptr(), _lib.i64_array(dq.stride())
     args.dk, args.dk_stride = dk.data_ptr(), _lib.i64_array(dk.stride())
     args.dv, args.dv_stride = dv.data_ptr(), _lib.i64_array(dv.stride())
@@ -232,6 +242,9 @@ def dsqg_backward(dout, q, k, v, pos_bias, scale_embed, phase_base, phase_gain, 
     nbytes = lib.dwarf_dsqg_bwd_workspace_bytes(ctypes.byref(args))
     workspace = torch.empty(max(int(nbytes), 256), device=dev, dtype=torch.uint8)
     args.workspace, args.workspace_bytes = workspace.data_ptr(), workspace.numel()
+    paired = overlap and callable(dout)
+    dout = _kernel_rows((dout(workspace.data_ptr() if overlap else 0) if callable(dout) else dout).to(q.dtype))
+    args.dout, args.dout_stride = dout.data_ptr(), _lib.i64_array(dout.stride())
     stream = _stream(dev)
     if one_call:
         _lib.check(lib.dwarf_dsqg_bwd(ctypes.byref(args), stream), "dwarf_dsqg_bwd")
@@ -253,7 +266,8 @@ def dsqg_backward(dout, q, k, v, pos_bias, scale_embed, phase_base, phase_gain, 
         side.wait_event(fork)
         if ev:
             ev[3].record(side)
-        _lib.check(lib.dwarf_dsqg_bwd_delta(ctypes.byref(args), side.cuda_stream), "dwarf_dsqg_bwd_delta")
+        if not paired:
+            _lib.check(lib.dwarf_dsqg_bwd_delta(ctypes.byref(args), side.cuda_stream), "dwarf_dsqg_bwd_delta")
         if ev:
             ev[4].record(side)
         _lib.check(lib.dwarf_dsqg_bwd_dkdv(ctypes.byref(args), side.cuda_stream), "dwarf_dsqg_bwd_dkdv")

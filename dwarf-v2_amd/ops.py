@@ -4,7 +4,8 @@
 ``dwarf::dsqg_bwd_probed``, ``dwarf::ema_fwd``,
 ``dwarf::ema_bwd``, ``dwarf::phase_probe_fwd``, ``dwarf::phase_probe_bwd``,
 ``dwarf::npci_fwd``, ``dwarf::npci_bwd``, ``dwarf::packet_pool_fwd``,
-``dwarf::packet_pool_bwd``, ``dwarf::packet_fwd`` and ``dwarf::packet_bwd`` are
+``dwarf::packet_pool_bwd``, ``dwarf::packet_fwd``, ``dwarf::packet_bwd``,
+``dwarf::dsqg_block_fwd`` and ``dwarf::dsqg_block_bwd`` are
 custom ops with fake (shape-only) implementations, so ``torch.compile`` traces
 the DSQG, EMA, phase-probe, NPCI and InterferencePacket autograd Functions
 without graph breaks (the trainer
@@ -23,6 +24,7 @@ from typing import Optional
 
 import torch
 
+from . import block as _block
 from . import dsqg as _dsqg
 from . import ema as _ema
 from . import npci as _npci
@@ -118,6 +120,48 @@ def _dsqg_bwd_probed_fake(dout, q, k, v, pos_bias, scale_embed, phase_base, phas
     return (q.new_empty(q.shape), q.new_empty(k.shape), q.new_empty(v.shape),
             q.new_empty(pos_bias.shape, dtype=f32), q.new_empty(scale_embed.shape, dtype=f32),
             q.new_empty(phase_base.shape, dtype=f32), q.new_empty(phase_gain.shape, dtype=f32))
+
+
+# ---- the DSQG block between its projections ---------------------------------------------------
+@torch.library.custom_op("dwarf::dsqg_block_fwd", mutates_args=())
+def dsqg_block_fwd(qkvg: Tensor, pos_bias: Tensor, scale_embed: Tensor, phase_base: Tensor, phase_gain: Tensor,
+                   query_probes: Tensor, key_probes: Tensor, gain: Tensor, offsets: Tensor, heads: int, j_small: int,
+                   j_large: int, plane_shift: int, query_start: int, schedule: int
+                   ) -> tuple[Tensor, Tensor, Tensor, Tensor, Tensor]:
+    """(gated [B,N,D], out [B,N,H,64], lse [B,H,N] fp32, y, z [B,H,N,4] fp32) from the fused projection [B,N,4D]."""
+    return _block.block_forward(qkvg, pos_bias, scale_embed, phase_base, phase_gain, query_probes, key_probes, gain,
+                                offsets, heads, j_small, j_large, plane_shift, query_start, schedule)
+
+
+@dsqg_block_fwd.register_fake
+def _dsqg_block_fwd_fake(qkvg, pos_bias, scale_embed, phase_base, phase_gain, query_probes, key_probes, gain, offsets,
+                         heads, j_small, j_large, plane_shift, query_start, schedule):
+    B, N, D4 = qkvg.shape
+    f32 = torch.float32
+    return (qkvg.new_empty((B, N, D4 // 4)), qkvg.new_empty((B, N, heads, D4 // 4 // heads)),
+            qkvg.new_empty((B, heads, N), dtype=f32), qkvg.new_empty((B, heads, N, 4), dtype=f32),
+            qkvg.new_empty((B, heads, N, 4), dtype=f32))
+
+
+@torch.library.custom_op("dwarf::dsqg_block_bwd", mutates_args=())
+def dsqg_block_bwd(dgated: Tensor, qkvg: Tensor, pos_bias: Tensor, scale_embed: Tensor, phase_base: Tensor,
+                   phase_gain: Tensor, query_probes: Tensor, key_probes: Tensor, gain: Tensor, offsets: Tensor,
+                   out: Tensor, lse: Tensor, y: Tensor, z: Tensor, heads: int, j_small: int, j_large: int,
+                   plane_shift: int, query_start: int, schedule: int
+                   ) -> tuple[Tensor, Tensor, Tensor, Tensor, Tensor, Tensor]:
+    """(dqkvg, dpos_bias, dscale_embed, dphase_base, dphase_gain, dgain [H])."""
+    return _block.block_backward(dgated, qkvg, pos_bias, scale_embed, phase_base, phase_gain, query_probes, key_probes,
+                                 gain, offsets, out, lse, y, z, heads, j_small, j_large, plane_shift, query_start,
+                                 schedule)
+
+
+@dsqg_block_bwd.register_fake
+def _dsqg_block_bwd_fake(dgated, qkvg, pos_bias, scale_embed, phase_base, phase_gain, query_probes, key_probes, gain,
+                         offsets, out, lse, y, z, heads, j_small, j_large, plane_shift, query_start, schedule):
+    f32 = torch.float32
+    return (qkvg.new_empty(qkvg.shape), *(qkvg.new_empty(t.shape, dtype=f32)
+                                          for t in (pos_bias, scale_embed, phase_base, phase_gain)),
+            qkvg.new_empty((heads,), dtype=f32))
 
 
 # ---- EMA -------------------------------------------------------------------------------------

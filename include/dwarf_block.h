@@ -1,0 +1,60 @@
+/*
+ * Entry points for the DSQG block around the attention op (libdwarf_dsqg.so,
+ * gfx950): the per-head gain and content gate after the attention, forward and
+ * backward.  Conventions (status codes, strides in elements, dwarf_stream_t)
+ * are those of dwarf_dsqg.h.
+ */
+#ifndef DWARF_BLOCK_H
+#define DWARF_BLOCK_H
+
+#include "dwarf_dsqg.h"
+
+#ifdef __cplusplus
+extern "C" {
+#endif
+
+/*
+ * gated[b,n,h*64+d] = bf16((out[b,h,n,d] * gain[h]) * bf16(sigmoid(gate[b,n,h*64+d]))), the products in
+ * fp32: the block's if_gain and content gate (dsqg:3278-3284) under bf16 autocast.  out [B,H,N,64], gate and
+ * gated [B,N,H*64], all bf16 with unit last stride and 16-byte aligned rows; gain [H] fp32.
+ */
+typedef struct {
+  int32_t B, H, N;
+  const void* out; int64_t out_stride[4];
+  const float* gain;
+  const void* gate; int64_t gate_stride[3];
+  void* gated; int64_t gated_stride[3];
+} dwarf_head_gate_fwd_args;
+
+int dwarf_head_gate_fwd(const dwarf_head_gate_fwd_args* args, dwarf_stream_t stream);
+
+/*
+ * The gradients autograd forms for that expression, with its roundings: with s = bf16(sigmoid(gate)) and
+ * dm = dgated * s, dout = bf16(dm * gain), dgate = bf16(bf16(dgated * out * gain) * (1 - s) * s) and
+ * dgain[h] = sum of dm * out in fp32 in a fixed order.  fwd.gated is not used.
+ *
+ * delta_pairs (may be NULL): [B,H,N] pairs (sum_d dout * out, lse * log2 e; +inf where lse is -inf or
+ * n < query_start), what dwarf_dsqg_bwd_delta writes at the start of the DSQG backward's workspace; a caller
+ * that passes the workspace's address here runs its stages under DWARF_SCHED_DELTA_STAGE without that launch.
+ * lse [B,H,N] fp32 is read then.
+ */
+typedef struct {
+  dwarf_head_gate_fwd_args fwd;
+  const void* dgated; int64_t dgated_stride[3];
+  void* dout; int64_t dout_stride[4];
+  void* dgate; int64_t dgate_stride[3];
+  float* dgain;
+  const float* lse; int64_t lse_stride[3];
+  int32_t query_start;
+  float* delta_pairs;
+  void* workspace; size_t workspace_bytes;   /* 16-byte aligned */
+} dwarf_head_gate_bwd_args;
+
+size_t dwarf_head_gate_bwd_workspace_bytes(const dwarf_head_gate_bwd_args* args);
+int dwarf_head_gate_bwd(const dwarf_head_gate_bwd_args* args, dwarf_stream_t stream);
+
+#ifdef __cplusplus
+}
+#endif
+
+#endif /* DWARF_BLOCK_H */

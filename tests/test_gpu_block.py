@@ -174,3 +174,109 @@ def test_block_forward_fp32_crop_and_kv_inject(pkg, device):
     kv_inject through the NPCI rotation of the live key/value prefix: out, dx and every parameter gradient
     within 1e-5 relative of the float64 restatement."""
     _compare(pkg, device, "far", True, torch.float32, 1e-5, 1e-5)
+
+
+def _ulp(x):
+    """bf16 spacing at |x|."""
+    return torch.exp2(torch.floor(torch.log2(x.abs().clamp_min(1e-30)))) * 2.0 ** -7
+
+
+@pytest.mark.parametrize("B,H,N,pairs", [(1, 1, 1, False), (2, 3, 37, True), (1, 40, 33, False), (3, 8, 700, True)])
+def test_head_gate_against_the_expression(pkg, device, B, H, N, pairs):
+    """The gain-and-gate launches against the expression in float64 with its bf16 roundings: one item, heads that do
+    not divide a workgroup's items (3), more heads than items (40), several grid strides; the gate and dout as strided
+    views.  bf16 results within one spacing (a float32 product on the other side of a rounding boundary; a bf16
+    sigmoid likewise moves one spacing, so two for what it multiplies); dgain: B N 64 float32 products, bounded by
+    2e-6 of the sum of their magnitudes.  The (delta, lse) pairs against the sum over the rounded dout."""
+    block = pkg.block
+    g = torch.Generator().manual_seed(7 * N + H)
+    D = 64 * H
+    qkvg = torch.randn(B, N, 4 * D, generator=g).to(torch.bfloat16).to(device)
+    gate = qkvg[..., 3 * D:]
+    out = torch.randn(B, N, H, 64, generator=g).to(torch.bfloat16).to(device).permute(0, 2, 1, 3)
+    gain = (1 + 0.3 * torch.randn(H, generator=g)).to(device)
+    dg = torch.randn(B, N, D, generator=g).to(torch.bfloat16).to(device)
+    lse = torch.randn(B, H, N, generator=g).to(device)
+    lse[:, :, :1] = float("-inf")
+    got = block.head_gate_forward(out, gain, gate)
+    dgate = torch.empty_like(qkvg)[..., 3 * D:]
+    ws = torch.full((B, H, N, 2), float("nan"), device=device)
+    dout, dgain = block.head_gate_backward(dg, out, gain, gate, dgate, lse=lse, query_start=2,
+                                           pairs=ws.data_ptr() if pairs else 0)
+    torch.cuda.synchronize()
+
+    def r16(t):
+        return t.to(torch.bfloat16).double()
+
+    o = out.double().cpu().permute(0, 2, 1, 3).reshape(B, N, D)
+    s, d, gn = r16(torch.sigmoid(gate.double().cpu())), dg.double().cpu(), gain.double().cpu().repeat_interleave(64)
+    want = o * gn * s
+    assert ((got.double().cpu() - want).abs() <= 2 * _ulp(want)).all()
+    wd = d * s * gn
+    gd = dout.double().cpu().permute(0, 2, 1, 3).reshape(B, N, D)
+    assert ((gd - wd).abs() <= 2 * _ulp(wd)).all()
+    ds = r16(d * o * gn)
+    wg = ds * (1 - s) * s
+    # dgate multiplies s and 1 - s, each a bf16 spacing off at most: 2^-7 (1 - s) + 2^-8 s of ds beside its own rounding
+    assert ((dgate.double().cpu() - wg).abs() <= 2 * _ulp(wg) + ds.abs() * 2.0 ** -7).all()
+    wgain = (d * s * o).reshape(B * N, H, 64)
+    err = (dgain.double().cpu() - wgain.sum((0, 2))).abs()
+    # a sigmoid on the other side of its rounding boundary (one in 10^4) shifts its own term by 2^-8
+    assert (err <= 2e-6 * wgain.abs().sum((0, 2)) + 2.0 ** -8 * wgain.abs().amax((0, 2))).all()
+    if pairs:
+        p = ws.double().cpu()
+        wdelta = (gd * o).reshape(B, N, H, 64).sum(-1).permute(0, 2, 1)
+        bound = 1e-6 * (gd * o).abs().reshape(B, N, H, 64).sum(-1).permute(0, 2, 1)
+        assert ((p[..., 0] - wdelta).abs() <= bound).all()
+        live = (torch.arange(N) >= 2) & torch.isfinite(lse.cpu())
+        want2 = torch.where(live, lse.double().cpu() * 1.4426950408889634, torch.tensor(float("inf"), dtype=torch.double))
+        assert torch.equal(torch.isinf(p[..., 1]), torch.isinf(want2))
+        assert ((p[..., 1] - want2).abs()[live] <= 1e-6).all() if live.any() else True
+
+
+@pytest.mark.parametrize("H,N,lattice,ones", [(3, 65, "third1", False), (8, 301, "third2", True), (4, 130, "canonical", False)])
+def test_block_as_one_node_equals_the_composed_block(pkg, device, H, N, lattice, ones):
+    """The one-node block (bf16 autocast) against the composed one, which a forward hook on the output projection
+    selects: out, dx and every parameter gradient.  Both round the same products, in the same places; the bars are
+    two bf16 spacings of the largest magnitude (2^-7), for sums over tokens of terms rounded a spacing apart."""
+    offsets = list(pkg.ALL_OFFSETS) if lattice == "canonical" else list(pkg.lattice.build_offset_groups(2048)[int(lattice[-1])])
+    js = sum(d <= 28 for d in offsets)
+    blk = StandInBlock(64 * H, H, offsets, js, 4, 64, seed=H + N).to(device)
+    g = torch.Generator().manual_seed(N)
+    x = torch.randn(2, N, 64 * H, generator=g).to(torch.bfloat16).to(device).requires_grad_(True)
+    dy = torch.randn(2, N, 64 * H, generator=g).to(torch.bfloat16).to(device)
+    named = [(n, p) for n, p in blk.named_parameters() if p.requires_grad and not n.startswith("npci")]
+
+    def both():
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            out = pkg.dsqg_block_forward(blk, x)
+        loss = out.float().sum() if ones else (out * dy).float().sum()
+        return [out.detach()] + list(torch.autograd.grad(loss, [x] + [p for _, p in named]))
+
+    one = both()
+    blk.out_proj.register_forward_hook(lambda m, i, o: None)
+    composed = both()
+    for n, a, b in zip(["out", "x"] + [n for n, _ in named], one, composed):
+        assert a.dtype == b.dtype and a.shape == b.shape, n
+        scale = float(b.abs().max())
+        assert float((a.double() - b.double()).abs().max()) <= 2.0 ** -7 * scale, n
+
+
+def test_block_one_node_compiles(pkg, device):
+    """torch.compile traces the block's node with fullgraph and gives the eager bits."""
+    offsets = list(pkg.lattice.build_offset_groups(2048)[0])
+    blk = StandInBlock(256, 4, offsets, sum(d <= 28 for d in offsets), 2, 64, seed=3).to(device)
+    x = torch.randn(2, 96, 256, generator=torch.Generator().manual_seed(1)).to(torch.bfloat16).to(device)
+
+    def step(inp):
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            return pkg.dsqg_block_forward(blk, inp)
+
+    a, b = x.clone().requires_grad_(True), x.clone().requires_grad_(True)
+    ea = step(a)
+    eb = torch.compile(step, fullgraph=True)(b)
+    ea.float().sum().backward()
+    eb.float().sum().backward()
+    scale = float(ea.abs().max())
+    assert float((ea - eb).abs().max()) <= 2.0 ** -7 * scale
+    assert float((a.grad - b.grad).abs().max()) <= 2.0 ** -6 * float(a.grad.abs().max())
