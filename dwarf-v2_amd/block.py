@@ -164,10 +164,12 @@ class _DSQGBlockFn(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, qkvg, pos_bias, scale_embed, phase_base, phase_gain, gain, query_probes, key_probes, offsets_dev,
-                heads, j_small, j_large, plane_shift, query_start, schedule):
-        ctx.args = (int(heads), int(j_small), int(j_large), int(plane_shift), int(query_start), int(schedule))
+                heads, j_small, j_large, plane_shift, query_start, schedule, bwd_schedule):
+        args = (int(heads), int(j_small), int(j_large), int(plane_shift), int(query_start))
+        ctx.args = (*args, int(bwd_schedule))
         gated, out, lse, y, z = torch.ops.dwarf.dsqg_block_fwd(qkvg, pos_bias, scale_embed, phase_base, phase_gain,
-                                                               query_probes, key_probes, gain, offsets_dev, *ctx.args)
+                                                               query_probes, key_probes, gain, offsets_dev, *args,
+                                                               int(schedule))
         ctx.save_for_backward(qkvg, pos_bias, scale_embed, phase_base, phase_gain, gain, query_probes, key_probes,
                               offsets_dev, out, lse, y, z)
         return gated
@@ -178,7 +180,7 @@ class _DSQGBlockFn(torch.autograd.Function):
         g = torch.ops.dwarf.dsqg_block_bwd(dgated, qkvg, pb, se, pbase, pgain, qp, kp, gain, offsets, out, lse, y, z,
                                            *ctx.args)
         dqkvg, dpb, dse, dpbase, dpgain, dgain = g
-        return (dqkvg, dpb, dse, dpbase, dpgain, dgain.reshape(gain.shape)) + (None,) * 9
+        return (dqkvg, dpb, dse, dpbase, dpgain, dgain.reshape(gain.shape)) + (None,) * 10
 
 
 def _plain_linear(m) -> bool:
@@ -212,7 +214,8 @@ def _gated_heads(block, proj: torch.Tensor, query_start: int) -> torch.Tensor:
         proj, block.pos_bias.float(), block.centered_scale_embed.float(), (block.phase_base * phase_gate).float(),
         (block.phase_gain * phase_gate).float(), block.if_gain.reshape(-1), qp, kp, block.offsets_dev, H,
         int(block.j_small), int(block.j_large), int(block.plane_shift), max(0, min(int(query_start), proj.shape[1])),
-        schedule_for(block.grouped_mode_id, bool(block.online_softmax)))
+        *(schedule_for(block.grouped_mode_id, bool(block.online_softmax), int(block.j_small), back)
+          for back in (False, True)))
 
 
 def _inject(block, k: torch.Tensor, v: torch.Tensor, kv_inject, key_end: int):

@@ -29,18 +29,25 @@ from .lattice import GROUPED_MODE_IDS, R_PLANES
 
 HEAD_DIM = 64
 _SLAB_MODES = (GROUPED_MODE_IDS["overlap_slab"], GROUPED_MODE_IDS["overlap_slab_bwd"])
-# Schedule of the baseline mode: the near band of the dQ and dK/dV launches on
-# the matrix cores (DWARF_SCHED_BAND) measured faster than the gather loops
-# alone at B15 H8 T2048 (dQ 271 vs 280-284 us, dK/dV 241 vs 262-265 us on one
-# box), so it is the default; 0 selects the gather loops alone.  The
-# overlap-slab modes always set it; online_softmax=False adds
-# DWARF_SCHED_TWO_PASS (the offline-softmax forward).
-DEFAULT_SCHEDULE = 1
+# Schedule of the baseline mode with many near offsets: the near band on the
+# matrix cores (DWARF_SCHED_BAND; dQ 234 vs 252 us and dK/dV 205 vs 232 at B15
+# H8 T2048, 17 near and 79 far offsets); 0 selects the gather loops alone.
+# The band costs the same however few offsets it holds, the gather loop by the
+# offset, so short bands are gathered (``schedule_for``).
+DEFAULT_SCHEDULE = _lib.DWARF_SCHED_BAND
+# Fewest near offsets from which the band is the faster one.  Band against gather in us, overlapped backward:
+# B15 T2048, 23 far: 6 near 269 / 239, 9 273 / 255, 10 271 / 263, 12 271 / 273, 17 278 / 305; 79 far: 9 454 / 438,
+# 10 450 / 450, 12 454 / 461; B4 T8192, 23 far: 9 354 / 336, 10 351 / 352, 12 355 / 361.  Forward, B15 T2048, 23 far:
+# 3 near 71 / 62, 6 68 / 67, 8 70 / 73, 10 69 / 78; B4 T8192, 79 far: 6 208 / 209, 8 210 / 210, 10 207 / 214.
+BAND_MIN_FORWARD, BAND_MIN_BACKWARD = 7, 11
 
 
-def schedule_for(grouped_mode_id: int, online_softmax: bool) -> int:
-    """DWARF_SCHED_* flags for the reference's mode arguments (dsqg:2271-2314, 2394, 2470)."""
-    sched = DEFAULT_SCHEDULE
+def schedule_for(grouped_mode_id: int, online_softmax: bool, j_small: int | None = None, backward: bool = False) -> int:
+    """DWARF_SCHED_* flags for the reference's mode arguments (dsqg:2271-2314, 2394, 2470).  The overlap-slab
+    modes always set DWARF_SCHED_BAND; the baseline mode sets it where ``j_small`` near offsets are enough for it
+    (None: always).  online_softmax=False adds DWARF_SCHED_TWO_PASS (the offline-softmax forward)."""
+    least = BAND_MIN_BACKWARD if backward else BAND_MIN_FORWARD
+    sched = DEFAULT_SCHEDULE if j_small is None or j_small >= least else 0
     if int(grouped_mode_id) in _SLAB_MODES:
         sched |= _lib.DWARF_SCHED_BAND
     if not online_softmax:
@@ -132,7 +139,7 @@ def dsqg_forward(q, k, v, pos_bias, scale_embed, phase_base, phase_gain, y_pre, 
 
     ``events``: optional (start, end) torch.cuda.Event pair recorded around the
     launch on the current stream.  ``schedule``: DWARF_SCHED_* flags (None: the
-    default schedule, ``DEFAULT_SCHEDULE``).  ``query_probes`` (bf16 only):
+    baseline mode's, ``schedule_for``).  ``query_probes`` (bf16 only):
     normalised [4,64] fp32 probes; the kernel forms y from q itself (y_pre is
     not read and may be None) and the call returns (out, lse, y) with y
     [B,H,N,4] fp32.
@@ -145,7 +152,7 @@ def dsqg_forward(q, k, v, pos_bias, scale_embed, phase_base, phase_gain, y_pre, 
     args = _lib.DsqgFwdArgs()
     _fill_fwd(args, q, k, v, pos_bias, scale_embed, phase_base, phase_gain, y_pre, z_pre, offsets_dev,
               j_small, j_large, plane_shift, query_start, out, lse, se_round=q.dtype != torch.float32,
-              schedule=DEFAULT_SCHEDULE if schedule is None else schedule)
+              schedule=schedule_for(0, True, j_small) if schedule is None else schedule)
     y = None
     if query_probes is not None:
         y = torch.empty((B, H, N, R_PLANES), device=q.device, dtype=torch.float32)
@@ -217,7 +224,8 @@ def dsqg_backward(dout, q, k, v, pos_bias, scale_embed, phase_base, phase_gain, 
     dz = torch.empty(z_pre.shape, device=dev, dtype=torch.float32) if key_probes is None else None
     # the delta-stage flag is this function's to set: it only holds when the delta launch runs
     # below, and on its own it would leave dK/dV reading (delta, lse) pairs no stage wrote
-    schedule = (DEFAULT_SCHEDULE if schedule is None else int(schedule)) & ~_lib.DWARF_SCHED_DELTA_STAGE
+    schedule = schedule_for(0, True, j_small, True) if schedule is None else int(schedule)
+    schedule &= ~_lib.DWARF_SCHED_DELTA_STAGE
     args = _lib.DsqgBwdArgs()
     _fill_fwd(args.fwd, q, k, v, pos_bias, scale_embed, phase_base, phase_gain, y_pre, z_pre, offsets_dev,
               j_small, j_large, plane_shift, query_start, out, lse, se_round=q.dtype != torch.float32,
@@ -344,7 +352,7 @@ class _DSQGV18GroupedFn(torch.autograd.Function):
         N = q.shape[2]
         query_start = max(0, min(int(query_start), N))
         _check_call(q, k, v, y_pre.shape, z_pre.shape, j_val, j_small, j_large, offsets_dev, grouped_mode_id)
-        schedule = schedule_for(grouped_mode_id, bool(online_softmax))
+        schedule = schedule_for(grouped_mode_id, bool(online_softmax), int(j_small))
         out, lse = torch.ops.dwarf.dsqg_fwd(q, k, v, pos_bias, scale_embed, phase_base, phase_gain, y_pre, z_pre,
                                             offsets_dev, int(j_small), int(j_large), int(plane_shift), query_start,
                                             schedule)
@@ -352,7 +360,7 @@ class _DSQGV18GroupedFn(torch.autograd.Function):
                               out, lse, offsets_dev)
         ctx.j_small, ctx.j_large = int(j_small), int(j_large)
         ctx.plane_shift, ctx.query_start = int(plane_shift), query_start
-        ctx.schedule = schedule
+        ctx.schedule = schedule_for(grouped_mode_id, bool(online_softmax), int(j_small), True)
         return out
 
     @staticmethod
@@ -429,7 +437,7 @@ class _DSQGProbedFn(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, q, k, v, pos_bias, scale_embed, phase_base, phase_gain, query_probes, key_probes, offsets_dev,
-                j_small, j_large, plane_shift, query_start, schedule):
+                j_small, j_large, plane_shift, query_start, schedule, bwd_schedule=None):
         N = q.shape[2]
         z_pre = torch.ops.dwarf.phase_probe_fwd(k, key_probes, 0, N)
         out, lse, y_pre = torch.ops.dwarf.dsqg_fwd_probed(q, k, v, pos_bias, scale_embed, phase_base, phase_gain,
@@ -438,7 +446,8 @@ class _DSQGProbedFn(torch.autograd.Function):
                                                           int(schedule))
         ctx.save_for_backward(q, k, v, pos_bias, scale_embed, phase_base, phase_gain, query_probes, key_probes,
                               y_pre, z_pre, out, lse, offsets_dev)
-        ctx.args = (int(j_small), int(j_large), int(plane_shift), int(query_start), int(schedule))
+        ctx.args = (int(j_small), int(j_large), int(plane_shift), int(query_start),
+                    int(schedule if bwd_schedule is None else bwd_schedule))
         return out
 
     @staticmethod
@@ -449,7 +458,7 @@ class _DSQGProbedFn(torch.autograd.Function):
             dout, q, k, v, pos_bias, scale_embed, phase_base, phase_gain, qp, kp, y_pre, z_pre, offsets, out, lse,
             *ctx.args)
         return (dq, dk.to(k.dtype), dv.to(v.dtype), dpb.to(pos_bias.dtype), dse.to(scale_embed.dtype),
-                dpbase.to(phase_base.dtype), dpgain.to(phase_gain.dtype)) + (None,) * 8
+                dpbase.to(phase_base.dtype), dpgain.to(phase_gain.dtype)) + (None,) * 9
 
 
 def dsqg_attention_with_probes(
@@ -500,5 +509,6 @@ def dsqg_attention_with_probes(
     output = _DSQGProbedFn.apply(
         qb, kb, vb, pos_bias.float(), scale_embed.float(), phase_base.float(), phase_gain.float(),
         qp.detach().to(q.device), kp.detach().to(q.device), offsets_dev, int(j_small), int(j_large), int(plane_shift),
-        max(0, min(int(query_start), N)), schedule_for(grouped_mode_id, bool(online_softmax)))
+        max(0, min(int(query_start), N)), *(schedule_for(grouped_mode_id, bool(online_softmax), int(j_small), back)
+                                            for back in (False, True)))
     return output if output.dtype == original_dtype else output.to(original_dtype)

@@ -277,6 +277,22 @@ def test_band_lattice_edges(pkg, device):
             assert max_abs(grads[n], rg[n]) < BF16_ABS, (offsets, n, max_abs(grads[n], rg[n]))
 
 
+@pytest.mark.parametrize("near", [6, 7, 10, 11])
+def test_default_schedule_by_near_offsets(pkg, device, near):
+    """The baseline mode on either side of the counts at which the forward and the backward turn from the gather
+    loops to the near band (a forward with the band and a backward without in between), against the oracle."""
+    full = lattice(pkg)
+    offsets = full[17 - near:17] + full[17:40]
+    x = make_inputs(1, 3, 3, 530, offsets, near, seed=200 + near, dtype=torch.bfloat16, plane_shift=3, gain_std=4.0)
+    dout = torch.randn(1, 3, 530, 64, generator=torch.Generator().manual_seed(201)).to(torch.bfloat16)
+    qs = min(offsets)
+    out, grads = gpu_fwd_bwd(pkg, x, offsets, near, 3, qs, dout, device)
+    ro, _, rg = oracle_fwd_bwd(x, offsets, near, 3, qs, dout.float(), round_se=True)
+    assert max_abs(out, ro) < BF16_ABS
+    for n in NAMES:
+        assert max_abs(grads[n], rg[n]) < BF16_ABS, (n, max_abs(grads[n], rg[n]))
+
+
 def _raw_step(pkg, d, off, dout, overlap, qs=1, one_call=False):
     out, lse = pkg.dsqg_forward(d["q"], d["k"], d["v"], d["pos_bias"], d["scale_embed"], d["phase_base"],
                                 d["phase_gain"], d["y_pre"], d["z_pre"], off, 17, 79, 2, qs)

@@ -181,6 +181,21 @@ def test_custom_ops_default_to_the_python_schedule(pkg):
     assert inspect.signature(ops._dsqg_fwd_fake).parameters["schedule"].default == dsqg.DEFAULT_SCHEDULE
 
 
+def test_schedule_by_mode_and_near_offsets(pkg):
+    """The band is set for the overlap-slab modes always, for the baseline mode from the counts at which it is the
+    faster schedule, and where the count is not known; the offline softmax flag is independent of it."""
+    dsqg = importlib.import_module("dwarf-v2_amd.dsqg")
+    L = pkg._lib
+    for back, least in ((False, dsqg.BAND_MIN_FORWARD), (True, dsqg.BAND_MIN_BACKWARD)):
+        for js in range(18):
+            for online in (True, False):
+                two = 0 if online else L.DWARF_SCHED_TWO_PASS
+                assert dsqg.schedule_for(0, online, js, back) == two | (L.DWARF_SCHED_BAND if js >= least else 0)
+                assert dsqg.schedule_for(1, online, js, back) == dsqg.schedule_for(3, online, js, back) \
+                    == two | L.DWARF_SCHED_BAND
+    assert dsqg.schedule_for(0, True) == dsqg.DEFAULT_SCHEDULE == L.DWARF_SCHED_BAND
+
+
 def test_integration_guide_names_exist(pkg):
     """Every ``amd.<name>`` the drop-in guide tells a maintainer to bind exists in the package, so the
     rebinding it shows runs as written."""
