@@ -281,7 +281,8 @@ class PacketBwdArgs(ctypes.Structure):
 
 
 # ---- include/dwarf_block.h ----
-BLOCK_SYMBOLS = ("dwarf_head_gate_fwd", "dwarf_head_gate_bwd_workspace_bytes", "dwarf_head_gate_bwd")
+BLOCK_SYMBOLS = ("dwarf_normalize_probes", "dwarf_dsqg_bwd_two_streams", "dwarf_head_gate_fwd",
+                 "dwarf_head_gate_bwd_workspace_bytes", "dwarf_head_gate_bwd")
 
 
 class HeadGateFwdArgs(ctypes.Structure):
@@ -396,6 +397,10 @@ def load() -> ctypes.CDLL:
     lib.dwarf_packet_bwd_workspace_bytes.argtypes = [POINTER(PacketBwdArgs)]
     lib.dwarf_packet_bwd.restype = c_int
     lib.dwarf_packet_bwd.argtypes = [POINTER(PacketBwdArgs), c_void_p]
+    lib.dwarf_normalize_probes.restype = c_int
+    lib.dwarf_normalize_probes.argtypes = [c_void_p, c_void_p, c_void_p, c_void_p]
+    lib.dwarf_dsqg_bwd_two_streams.restype = c_int
+    lib.dwarf_dsqg_bwd_two_streams.argtypes = [POINTER(DsqgBwdArgs), c_int32, c_void_p, c_void_p]
     lib.dwarf_head_gate_fwd.restype = c_int
     lib.dwarf_head_gate_fwd.argtypes = [POINTER(HeadGateFwdArgs), c_void_p]
     lib.dwarf_head_gate_bwd_workspace_bytes.restype = c_size_t

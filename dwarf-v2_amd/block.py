@@ -39,7 +39,7 @@ import torch.nn.functional as F
 
 from . import _lib
 from .dsqg import (HEAD_DIM, _check_call, _planes, _rows_ok, _stream, dsqg_attention_with_probes, dsqg_backward,
-                   dsqg_forward, normalize_inputs, schedule_for)
+                   dsqg_forward, normalize_inputs, normalized_probe_banks, schedule_for)
 from .npci import npci_rotate
 from .probe import probe_forward
 
@@ -207,8 +207,7 @@ def _gated_heads(block, proj: torch.Tensor, query_start: int) -> torch.Tensor:
     q, k, v, _ = proj.split(proj.shape[-1] // 4, dim=-1)
     q, k, v = (_heads(t, H) for t in (q, k, v))
     _check_call(q, k, v, None, None, block.j_val, block.j_small, block.j_large, block.offsets_dev, block.grouped_mode_id)
-    qp = F.normalize(block.query_probes.detach().float(), dim=-1).to(proj.device)
-    kp = F.normalize(block.key_probes.detach().float(), dim=-1).to(proj.device)
+    qp, kp = normalized_probe_banks(block.query_probes, block.key_probes, proj.device)
     phase_gate = torch.sigmoid(block.phase_gate)[:, None, None]
     return _DSQGBlockFn.apply(
         proj, block.pos_bias.float(), block.centered_scale_embed.float(), (block.phase_base * phase_gate).float(),

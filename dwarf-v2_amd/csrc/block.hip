@@ -1,5 +1,6 @@
-// The DSQG block's per-head gain and content gate (dsqg:3278-3284), forward
-// and backward, one pass each.  PyTorch's chain for the same is six launches
+// The DSQG block around the attention: its normalised phase probes, and its
+// per-head gain and content gate (dsqg:3278-3284), forward and backward, one
+// pass each.  PyTorch's chain for the same is six launches
 // forward (fp32 product, permute copy, sigmoid, product, cast) and nine
 // backward, most of them on fp32 tensors.
 #include "common.h"
@@ -124,6 +125,17 @@ __global__ __launch_bounds__(kBlock) void head_gate_gain_kernel(const float* __r
   if (threadIdx.x == 0) dgain[blockIdx.x] = (s_sum[0] + s_sum[1]) + (s_sum[2] + s_sum[3]);
 }
 
+// A wave per probe row (PyTorch's normalize of the two banks is eight launches,
+// 20 us of the stream).
+__global__ __launch_bounds__(8 * kWave) void normalize_probes_kernel(const float* __restrict__ q,
+                                                                     const float* __restrict__ k,
+                                                                     float* __restrict__ out) {
+  const int row = threadIdx.x / kWave, d = threadIdx.x % kWave;
+  const float x = (row < kPlanes ? q + row * kHeadDim : k + (row - kPlanes) * kHeadDim)[d];
+  const float ss = __shfl(wave_sum_to_last(x * x), kWave - 1);
+  out[row * kHeadDim + d] = __fdiv_rn(x, fmaxf(__fsqrt_rn(ss), 1e-12f));
+}
+
 // Workgroups whose item slots are a multiple of H.
 unsigned gate_bwd_wgs(int H, unsigned items) {
   int a = H, b = kItems;   // H / gcd(H, kItems)
@@ -139,6 +151,11 @@ unsigned gate_bwd_wgs(int H, unsigned items) {
 size_t head_gate_bwd_workspace(const dwarf_head_gate_bwd_args& a) {
   return static_cast<size_t>(gate_bwd_wgs(a.fwd.H, static_cast<unsigned>(a.fwd.B) * a.fwd.N * a.fwd.H)) * kItems *
          sizeof(float);
+}
+
+hipError_t launch_normalize_probes(const float* q, const float* k, float* out, hipStream_t stream) {
+  hipLaunchKernelGGL(normalize_probes_kernel, dim3(1), dim3(8 * kWave), 0, stream, q, k, out);
+  return hipGetLastError();
 }
 
 hipError_t launch_head_gate_fwd(const dwarf_head_gate_fwd_args& a, hipStream_t stream) {

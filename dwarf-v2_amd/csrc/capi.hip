@@ -44,6 +44,7 @@ hipError_t launch_interference_packet_fwd(const dwarf_packet_fwd_args& a, hipStr
 hipError_t launch_interference_packet_bwd(const dwarf_packet_bwd_args& a, hipStream_t stream);
 hipError_t launch_phase_probe_fwd(const dwarf_phase_probe_fwd_args& a, hipStream_t stream);
 hipError_t launch_phase_probe_bwd(const dwarf_phase_probe_bwd_args& a, hipStream_t stream);
+hipError_t launch_normalize_probes(const float* q, const float* k, float* out, hipStream_t stream);
 size_t head_gate_bwd_workspace(const dwarf_head_gate_bwd_args& a);
 hipError_t launch_head_gate_fwd(const dwarf_head_gate_fwd_args& a, hipStream_t stream);
 hipError_t launch_head_gate_bwd(const dwarf_head_gate_bwd_args& a, hipStream_t stream);
@@ -725,7 +726,45 @@ int dwarf_dsqg_q6_decode_noalloc(const dwarf_dsqg_q6_decode_args* args, dwarf_st
                     "dwarf_dsqg_q6_decode_noalloc");
 }
 
-// ---- the DSQG block's gain and gate -----------------------------------------
+// ---- the DSQG block around the attention ------------------------------------
+int dwarf_normalize_probes(const float* query_probes, const float* key_probes, float* out, dwarf_stream_t stream) {
+  if (!query_probes || !key_probes || !out) return fail(DWARF_ERR_INVALID_ARGUMENT, "a probe bank or out is NULL");
+  return hip_status(dwarf::launch_normalize_probes(query_probes, key_probes, out, reinterpret_cast<hipStream_t>(stream)),
+                    "dwarf_normalize_probes");
+}
+
+int dwarf_dsqg_bwd_two_streams(const dwarf_dsqg_bwd_args* args, int32_t pairs_ready, dwarf_stream_t stream,
+                               dwarf_stream_t side) {
+  if (!args) return fail(DWARF_ERR_INVALID_ARGUMENT, "args is NULL");
+  if (!(args->fwd.schedule & DWARF_SCHED_DELTA_STAGE))
+    return fail(DWARF_ERR_INVALID_ARGUMENT, "dwarf_dsqg_bwd_two_streams needs DWARF_SCHED_DELTA_STAGE");
+  const hipStream_t main_s = reinterpret_cast<hipStream_t>(stream), side_s = reinterpret_cast<hipStream_t>(side);
+  hipEvent_t fork = nullptr, join = nullptr;
+  hipError_t e = hipEventCreateWithFlags(&fork, hipEventDisableTiming);
+  if (e == hipSuccess) e = hipEventCreateWithFlags(&join, hipEventDisableTiming);
+  if (e == hipSuccess) e = hipEventRecord(fork, main_s);
+  int rc = e == hipSuccess ? DWARF_OK : hip_status(e, "dwarf_dsqg_bwd_two_streams");
+  if (rc == DWARF_OK) {
+    // dQ goes first: its persistent workgroups take their two slots per CU before dK/dV's thousands fill the rest
+    // (the other way round dQ waits for dK/dV to drain and the two barely overlap)
+    rc = dwarf_dsqg_bwd_dq(args, stream);
+    if (rc == DWARF_OK && (e = hipStreamWaitEvent(side_s, fork, 0)) != hipSuccess)
+      rc = hip_status(e, "dwarf_dsqg_bwd_two_streams");
+    if (rc == DWARF_OK) {
+      if (!pairs_ready) rc = dwarf_dsqg_bwd_delta(args, side);
+      if (rc == DWARF_OK) rc = dwarf_dsqg_bwd_dkdv(args, side);
+      if (rc == DWARF_OK) rc = dwarf_dsqg_bwd_params(args, stream);
+      e = hipEventRecord(join, side_s);
+      if (e == hipSuccess) e = hipStreamWaitEvent(main_s, join, 0);
+      if (e != hipSuccess && rc == DWARF_OK) rc = hip_status(e, "dwarf_dsqg_bwd_two_streams");
+    }
+  }
+  // an event in use is released when the work that records and waits for it has passed
+  if (fork) (void)hipEventDestroy(fork);
+  if (join) (void)hipEventDestroy(join);
+  return rc;
+}
+
 static int check_gate(const dwarf_head_gate_fwd_args& a) {
   if (a.B < 0 || a.H <= 0 || a.N < 0) return fail(DWARF_ERR_INVALID_ARGUMENT, "bad sizes B=%d H=%d N=%d", a.B, a.H, a.N);
   // the kernels number (b, n, h) with 32 bits, one grid stride of slack above

@@ -176,6 +176,14 @@ def _side_stream(device: torch.device) -> torch.cuda.Stream:
     return _SIDE_STREAMS[key]
 
 
+def _worth_two_streams(q: torch.Tensor, J: int) -> bool:
+    """Whether the backward's stages gain from two streams: by 64-query tiles x offsets.  Captured backward, two
+    streams against one in us: 16 tiles x 96 37.5 / 36.0, 80 x 29 33.7 / 31.4, 64 x 96 43 / 48, 128 x 96 52 / 63,
+    256 x 29 45 / 52, 256 x 96 75 / 105; an eager call also pays the host for the two events."""
+    B, H, N, _ = q.shape
+    return B * H * ((N + 63) // 64) * J >= 4096
+
+
 def dsqg_backward(dout, q, k, v, pos_bias, scale_embed, phase_base, phase_gain, y_pre, z_pre, offsets_dev,
                   out, lse, j_small, j_large, plane_shift=0, query_start=0, *, events=None, schedule=None,
                   overlap=None, one_call=False, overlap_events=None, query_probes=None, key_probes=None,
@@ -187,7 +195,7 @@ def dsqg_backward(dout, q, k, v, pos_bias, scale_embed, phase_base, phase_gain, 
     current stream and returns it; given the address it also writes the (delta, lse) pairs there, and the
     delta stage's own launch is left out.
 
-    bf16 (``overlap`` None or True, no ``events``): the delta stage and dK/dV
+    bf16 (``overlap`` True, or None and more than a small grid; no ``events``): the delta stage and dK/dV
     run on a second stream beside dQ and the parameter gradients on the
     current stream, which waits for both (DWARF_SCHED_DELTA_STAGE); the two
     gather launches then share the CUs.  Otherwise, and for fp32, the dq,
@@ -242,7 +250,9 @@ def dsqg_backward(dout, q, k, v, pos_bias, scale_embed, phase_base, phase_gain, 
             raise ValueError("events time the stages of separate calls; one_call runs them in one")
         overlap = bool(overlap) and q.dtype == torch.bfloat16
     else:
-        overlap = q.dtype == torch.bfloat16 and not events and (overlap is None or overlap)
+        if overlap is None:
+            overlap = bool(overlap_events) or _worth_two_streams(q, j_small + j_large)
+        overlap = q.dtype == torch.bfloat16 and not events and bool(overlap)
     if overlap_events and (one_call or not overlap):
         raise ValueError("overlap_events time the stages of the overlapped two-stream schedule")
     if overlap:
@@ -258,38 +268,34 @@ def dsqg_backward(dout, q, k, v, pos_bias, scale_embed, phase_base, phase_gain, 
         _lib.check(lib.dwarf_dsqg_bwd(ctypes.byref(args), stream), "dwarf_dsqg_bwd")
         return dq, dk, dv, dpb, dse, dpbase, dpgain, dy, dz
     if overlap:
-        main = torch.cuda.current_stream(dev)
+        # The current stream waits for the second one before the call returns, so whatever the allocator hands out
+        # again afterwards to work on the current stream (or once an event on it has passed) is no longer in use on
+        # either: no tensor here needs record_stream for the second stream.
         side = _side_stream(dev)
+        if not overlap_events:
+            with torch.cuda.device(dev):   # the call's events belong to the current device
+                _lib.check(lib.dwarf_dsqg_bwd_two_streams(ctypes.byref(args), int(paired), stream, side.cuda_stream),
+                           "dwarf_dsqg_bwd_two_streams")
+            return dq, dk, dv, dpb, dse, dpbase, dpgain, dy, dz
+        main = torch.cuda.current_stream(dev)
         fork = torch.cuda.Event()
         fork.record(main)
-        # dQ goes first: its persistent workgroups take their two slots per CU before
-        # dK/dV's thousands of workgroups fill the rest (the other way round dQ waits
-        # for dK/dV to drain and the two barely overlap)
         ev = overlap_events
-        if ev:
-            ev[0].record(main)
+        ev[0].record(main)
         _lib.check(lib.dwarf_dsqg_bwd_dq(ctypes.byref(args), stream), "dwarf_dsqg_bwd_dq")
-        if ev:
-            ev[1].record(main)
+        ev[1].record(main)
         side.wait_event(fork)
-        if ev:
+        try:
             ev[3].record(side)
-        if not paired:
-            _lib.check(lib.dwarf_dsqg_bwd_delta(ctypes.byref(args), side.cuda_stream), "dwarf_dsqg_bwd_delta")
-        if ev:
+            if not paired:
+                _lib.check(lib.dwarf_dsqg_bwd_delta(ctypes.byref(args), side.cuda_stream), "dwarf_dsqg_bwd_delta")
             ev[4].record(side)
-        _lib.check(lib.dwarf_dsqg_bwd_dkdv(ctypes.byref(args), side.cuda_stream), "dwarf_dsqg_bwd_dkdv")
-        if ev:
+            _lib.check(lib.dwarf_dsqg_bwd_dkdv(ctypes.byref(args), side.cuda_stream), "dwarf_dsqg_bwd_dkdv")
             ev[5].record(side)
-        _lib.check(lib.dwarf_dsqg_bwd_params(ctypes.byref(args), stream), "dwarf_dsqg_bwd_params")
-        if ev:
+            _lib.check(lib.dwarf_dsqg_bwd_params(ctypes.byref(args), stream), "dwarf_dsqg_bwd_params")
             ev[2].record(main)
-        main.wait_stream(side)
-        # memory the second stream used must not be handed out again before it is done
-        for t in (workspace, dk, dv, dz, dout, q, k, v, out, lse, y_pre, z_pre, pos_bias, scale_embed, phase_base,
-                  phase_gain, offsets_dev, key_probes):
-            if t is not None and t.is_cuda:
-                t.record_stream(side)
+        finally:
+            main.wait_stream(side)
         return dq, dk, dv, dpb, dse, dpbase, dpgain, dy, dz
     if events:
         events[0].record()
@@ -421,6 +427,24 @@ def dsqg_attention_v18_grouped(
     return output if output.dtype == original_dtype else output.to(original_dtype)
 
 
+def normalized_probe_banks(query_probes, key_probes, device):
+    """The two [4,64] probe banks row-normalised (dsqg:3231-3232), fp32 on ``device``, without gradient."""
+    qp, kp = query_probes.detach(), key_probes.detach()
+    if qp.shape != (R_PLANES, HEAD_DIM) or kp.shape != qp.shape:   # the kernels refuse other banks
+        return tuple(torch.nn.functional.normalize(p.float(), dim=-1).to(device) for p in (qp, kp))
+    return torch.ops.dwarf.normalize_probes(qp.to(device=device, dtype=torch.float32),
+                                            kp.to(device=device, dtype=torch.float32)).unbind(0)
+
+
+def normalize_probes(query_probes: torch.Tensor, key_probes: torch.Tensor) -> torch.Tensor:
+    """Raw launch: [2,4,64] fp32 normalised rows of two fp32 [4,64] banks on one GPU."""
+    qp, kp = query_probes.contiguous(), key_probes.contiguous()
+    out = torch.empty((2, R_PLANES, HEAD_DIM), device=qp.device, dtype=torch.float32)
+    _lib.check(_lib.load().dwarf_normalize_probes(qp.data_ptr(), kp.data_ptr(), out.data_ptr(), _stream(qp.device)),
+               "dwarf_normalize_probes")
+    return out
+
+
 # ---- the op with the block's phase-probe features inside the kernels -------------------------------------------
 class _DSQGProbedFn(torch.autograd.Function):
     """DSQG attention whose y and z come from probes inside the kernels (bf16).
@@ -489,12 +513,12 @@ def dsqg_attention_with_probes(
         )
     if not q.is_cuda:
         raise RuntimeError("DSQG HIP kernels were requested but the tensors are not on a GPU device")
-    qp = torch.nn.functional.normalize(query_probes.float(), dim=-1)
-    kp = torch.nn.functional.normalize(key_probes.float(), dim=-1)
-    probe_grad = torch.is_grad_enabled() and (qp.requires_grad or kp.requires_grad)
+    probe_grad = torch.is_grad_enabled() and (query_probes.requires_grad or key_probes.requires_grad)
     if q.dtype == torch.float32 or probe_grad:
         from .probe import phase_probe_features
 
+        qp = torch.nn.functional.normalize(query_probes.float(), dim=-1)
+        kp = torch.nn.functional.normalize(key_probes.float(), dim=-1)
         y_pre = phase_probe_features(q, qp)
         z_pre = phase_probe_features(k, kp)
         return dsqg_attention_v18_grouped(
@@ -506,9 +530,10 @@ def dsqg_attention_with_probes(
     qb, kb, vb = q.to(torch.bfloat16), k.to(torch.bfloat16), v.to(torch.bfloat16)
     N = q.shape[2]
     _check_call(qb, kb, vb, None, None, j_val, j_small, j_large, offsets_dev, grouped_mode_id)
+    qp, kp = normalized_probe_banks(query_probes, key_probes, q.device)
     output = _DSQGProbedFn.apply(
         qb, kb, vb, pos_bias.float(), scale_embed.float(), phase_base.float(), phase_gain.float(),
-        qp.detach().to(q.device), kp.detach().to(q.device), offsets_dev, int(j_small), int(j_large), int(plane_shift),
+        qp, kp, offsets_dev, int(j_small), int(j_large), int(plane_shift),
         max(0, min(int(query_start), N)), *(schedule_for(grouped_mode_id, bool(online_softmax), int(j_small), back)
                                             for back in (False, True)))
     return output if output.dtype == original_dtype else output.to(original_dtype)

@@ -5,6 +5,7 @@
 ``dwarf::ema_bwd``, ``dwarf::phase_probe_fwd``, ``dwarf::phase_probe_bwd``,
 ``dwarf::npci_fwd``, ``dwarf::npci_bwd``, ``dwarf::packet_pool_fwd``,
 ``dwarf::packet_pool_bwd``, ``dwarf::packet_fwd``, ``dwarf::packet_bwd``,
+``dwarf::normalize_probes``,
 ``dwarf::dsqg_block_fwd`` and ``dwarf::dsqg_block_bwd`` are
 custom ops with fake (shape-only) implementations, so ``torch.compile`` traces
 the DSQG, EMA, phase-probe, NPCI and InterferencePacket autograd Functions
@@ -120,6 +121,17 @@ def _dsqg_bwd_probed_fake(dout, q, k, v, pos_bias, scale_embed, phase_base, phas
     return (q.new_empty(q.shape), q.new_empty(k.shape), q.new_empty(v.shape),
             q.new_empty(pos_bias.shape, dtype=f32), q.new_empty(scale_embed.shape, dtype=f32),
             q.new_empty(phase_base.shape, dtype=f32), q.new_empty(phase_gain.shape, dtype=f32))
+
+
+@torch.library.custom_op("dwarf::normalize_probes", mutates_args=())
+def normalize_probes(query_probes: Tensor, key_probes: Tensor) -> Tensor:
+    """[2,4,64] fp32: the rows of two [4,64] probe banks over their norms."""
+    return _dsqg.normalize_probes(query_probes, key_probes)
+
+
+@normalize_probes.register_fake
+def _normalize_probes_fake(query_probes, key_probes):
+    return query_probes.new_empty((2, *query_probes.shape))
 
 
 # ---- the DSQG block between its projections ---------------------------------------------------

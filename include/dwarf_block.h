@@ -1,7 +1,8 @@
 /*
  * Entry points for the DSQG block around the attention op (libdwarf_dsqg.so,
- * gfx950): the per-head gain and content gate after the attention, forward and
- * backward.  Conventions (status codes, strides in elements, dwarf_stream_t)
+ * gfx950): the normalised phase probes, the backward's two streams in one
+ * call, and the per-head gain and content gate after the attention, forward
+ * and backward.  Conventions (status codes, strides in elements, dwarf_stream_t)
  * are those of dwarf_dsqg.h.
  */
 #ifndef DWARF_BLOCK_H
@@ -12,6 +13,21 @@
 #ifdef __cplusplus
 extern "C" {
 #endif
+
+/*
+ * out [2][4][64]: the rows of query_probes and key_probes (fp32 [4,64], contiguous) over max(norm, 1e-12)
+ * (dsqg:3231-3232).
+ */
+int dwarf_normalize_probes(const float* query_probes, const float* key_probes, float* out, dwarf_stream_t stream);
+
+/*
+ * The bf16 backward's stages on two streams: dq and params on `stream`, delta (left out where pairs_ready says
+ * that the workspace already holds the pairs, written on `stream`) and dkdv on `side`, which starts after what
+ * `stream` held before the call; `stream` then waits for `side`, also where a stage fails, so nothing that
+ * later work on `stream` reuses is still in use on `side`.  args->fwd.schedule holds DWARF_SCHED_DELTA_STAGE.
+ */
+int dwarf_dsqg_bwd_two_streams(const dwarf_dsqg_bwd_args* args, int32_t pairs_ready, dwarf_stream_t stream,
+                               dwarf_stream_t side);
 
 /*
  * gated[b,n,h*64+d] = bf16((out[b,h,n,d] * gain[h]) * bf16(sigmoid(gate[b,n,h*64+d]))), the products in

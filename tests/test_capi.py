@@ -309,3 +309,55 @@ def test_unknown_schedule_bits_refused_without_gpu(pkg, lib):
     for good in (0, L.DWARF_SCHED_BAND, L.DWARF_SCHED_TWO_PASS, L.DWARF_SCHED_DELTA_STAGE, 7):
         b.fwd.schedule = good
         assert lib.dwarf_dsqg_bwd_delta(ctypes.byref(b), None) == L.DWARF_ERR_WORKSPACE   # got past the flags
+
+
+BLOCK_HEADER = os.path.join(ROOT, "include", "dwarf_block.h")
+BLOCK_STRUCTS = {"dwarf_head_gate_fwd_args": "HeadGateFwdArgs", "dwarf_head_gate_bwd_args": "HeadGateBwdArgs"}
+
+
+def test_block_header_exports_and_layout(pkg, lib, tmp_path):
+    """include/dwarf_block.h: every declared function is exported and bound, and the ctypes structs mirror it."""
+    names = sorted(set(re.findall(r"^(?:int|size_t)\s+(dwarf_\w+)\s*\(", open(BLOCK_HEADER).read(), re.M)))
+    assert sorted(pkg._lib.BLOCK_SYMBOLS) == names
+    assert all(hasattr(lib, n) for n in names)
+    if shutil.which("gcc") is None:
+        pytest.skip("gcc not available")
+    lines = ['#include <stdio.h>', '#include <stddef.h>', '#include "dwarf_block.h"', "int main(void) {"]
+    for cname, pyname in BLOCK_STRUCTS.items():
+        lines.append(f'printf("{cname} sizeof %zu\\n", sizeof({cname}));')
+        lines += [f'printf("{cname} {f} %zu\\n", offsetof({cname}, {f}));' for f, _ in getattr(pkg._lib, pyname)._fields_]
+    src, exe = tmp_path / "layout.c", tmp_path / "layout"
+    src.write_text("\n".join(lines + ["return 0; }"]))
+    subprocess.run(["gcc", "-I", os.path.dirname(HEADER), str(src), "-o", str(exe)], check=True)
+    for line in subprocess.run([str(exe)], check=True, capture_output=True, text=True).stdout.splitlines():
+        cname, field, value = line.split()
+        struct = getattr(pkg._lib, BLOCK_STRUCTS[cname])
+        assert (ctypes.sizeof(struct) if field == "sizeof" else getattr(struct, field).offset) == int(value), line
+
+
+def test_block_entries_refuse_bad_calls_without_gpu(pkg, lib):
+    """The block entry points' host-side checks: NULL blocks, sizes past 32-bit item numbers, unaligned rows, a
+    short workspace, and two streams without the delta-stage flag."""
+    L = pkg._lib
+    bad = L.DWARF_ERR_INVALID_ARGUMENT
+    assert lib.dwarf_normalize_probes(None, None, None, None) == bad
+    assert lib.dwarf_dsqg_bwd_two_streams(None, 0, None, None) == bad
+    assert lib.dwarf_dsqg_bwd_two_streams(ctypes.byref(L.DsqgBwdArgs()), 0, None, None) == bad
+    assert lib.dwarf_head_gate_fwd(None, None) == bad and lib.dwarf_head_gate_bwd(None, None) == bad
+    a = L.HeadGateBwdArgs()
+    f = a.fwd
+    f.B, f.H, f.N = 1 << 12, 1 << 10, 1 << 10
+    assert lib.dwarf_head_gate_fwd(ctypes.byref(f), None) == L.DWARF_ERR_UNSUPPORTED
+    f.B, f.H, f.N = 2, 3, 5
+    f.out = f.gate = f.gated = f.gain = a.dgated = a.dout = a.dgate = a.dgain = 0x10000
+    rows, toks = L.i64_array((960, 64, 192, 1)), L.i64_array((960, 192, 1))
+    f.out_stride = a.dout_stride = rows
+    f.gate_stride = f.gated_stride = a.dgated_stride = a.dgate_stride = toks
+    a.workspace, a.workspace_bytes = 0x10000, 3 * 32 * 4 - 1      # H / gcd(H, 32) = 3 workgroups of 32 items
+    assert lib.dwarf_head_gate_bwd_workspace_bytes(ctypes.byref(a)) == 3 * 32 * 4
+    assert lib.dwarf_head_gate_bwd(ctypes.byref(a), None) == L.DWARF_ERR_WORKSPACE
+    a.delta_pairs = 0x10000                                       # needs lse
+    assert lib.dwarf_head_gate_bwd(ctypes.byref(a), None) == bad
+    f.gate = 0x10002
+    assert lib.dwarf_head_gate_fwd(ctypes.byref(f), None) == bad
+    assert b"16-byte" in lib.dwarf_last_error()

@@ -277,6 +277,26 @@ def test_band_lattice_edges(pkg, device):
             assert max_abs(grads[n], rg[n]) < BF16_ABS, (offsets, n, max_abs(grads[n], rg[n]))
 
 
+@pytest.mark.parametrize("B,h,N", [(1, 4, 130), (3, 8, 1500)])
+def test_two_stream_backward_leaves_nothing_in_use(pkg, device, B, h, N):
+    """The overlapped backward waits for its second stream before it returns: buffers that the allocator hands out
+    again straight after it (and that are written then, on the current stream) change no gradient.  Against the
+    serial backward, bit for bit, several calls in a row; default overlap on either side of its grid rule."""
+    offsets = lattice(pkg)
+    x = make_inputs(B, h, h, N, offsets, 17, seed=300, dtype=torch.bfloat16, plane_shift=2)
+    d = to_device(x, device)
+    off = torch.tensor(offsets, dtype=torch.int32, device=device)
+    dout = torch.randn(B, h, N, 64, generator=torch.Generator().manual_seed(3)).to(torch.bfloat16).to(device)
+    want = _raw_step(pkg, d, off, dout, False)
+    for overlap in (True, None):
+        for _ in range(4):
+            got = _raw_step(pkg, {n: t.clone() for n, t in d.items()}, off.clone(), dout.clone(), overlap)
+            trash = [torch.full((n,), float("nan"), device=device) for n in (1 << 16, 1 << 20, 1 << 22, 1 << 24)]
+            del trash
+            for a, b in zip(got, want):
+                assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize("near", [6, 7, 10, 11])
 def test_default_schedule_by_near_offsets(pkg, device, near):
     """The baseline mode on either side of the counts at which the forward and the backward turn from the gather

@@ -219,3 +219,20 @@ def test_probed_cfg2_as_benched(pkg, device):
         assert worst[n] < BF16_ABS, (n, worst[n])
     print("[probed] largest |gpu - oracle| (bar 2e-2): " + ", ".join(f"{n} {v:.2e}" for n, v in worst.items()),
           flush=True)
+
+
+def test_normalized_probe_banks(pkg, device):
+    """The one-launch probe normalisation against F.normalize in float64: a square root, a division and 64 summed
+    squares in float32 (2e-7 relative); a zero row stays zero; banks held as views or in bf16."""
+    g = torch.Generator().manual_seed(5)
+    qp, kp = torch.randn(8, 64, generator=g)[::2], 1e-3 * torch.randn(64, 4, generator=g).t()
+    qp = qp.clone()
+    qp[2] = 0
+    for dt in (torch.float32, torch.bfloat16):
+        a, b = qp.to(dt).to(device), kp.to(dt).to(device)
+        got = pkg.dsqg.normalized_probe_banks(a, b, a.device)
+        for y, p in zip(got, (a, b)):
+            want = torch.nn.functional.normalize(p.double(), dim=-1)
+            assert y.dtype == torch.float32 and not y.requires_grad
+            assert float((y.double() - want).abs().max()) <= 2e-7
+        assert not got[0][2].any()
