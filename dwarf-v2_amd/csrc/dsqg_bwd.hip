@@ -2,12 +2,12 @@
 // the kernels _compute_D_v18_grouped dsqg:1263-1289, _bwd_dq_v18_grouped
 // dsqg:1296-1488, _bwd_dkdv_v18_grouped dsqg:1734-1955).
 //
-// Launches on the caller's stream:
-//  1. dq kernel (dsqg_bwd_dq.hip), query-centric: delta, dQ, dY and one
-//     partial of dPB / dSE / dPhaseBase / dPhaseGain per workgroup.
-//  2. two reduce kernels: fixed-order sums of those partials (stage 1 over
-//     groups of 16 rows, stage 2 over the groups), so the parameter gradients
-//     are bitwise reproducible.
+// Launches on the caller's stream (bf16 here and in dsqg_bwd_dq.hip, fp32 in
+// dsqg_f32.hip):
+//  1. dq kernel, query-centric: dQ, dY, the dS matrix and dPhase partials.
+//  2. the dSE and dPB products of the dS matrix, then two reduce kernels:
+//     fixed-order sums of the partials (stage 1 over groups of rows, stage 2
+//     over the groups), so the parameter gradients are bitwise reproducible.
 //  3. dkdv kernel, key-centric.  For each key row m and each query head of
 //     its KV group, the pairs n = m + delta are revisited to accumulate dK,
 //     dV and dZ in registers; the GQA head sum happens in-kernel.
@@ -21,138 +21,6 @@ namespace {
 
 
 __host__ __device__ constexpr size_t align256(size_t x) { return (x + 255) & ~static_cast<size_t>(255); }
-
-template <typename T, int SHIFT, int L, bool FAST>
-__global__ __launch_bounds__(kBlock) void dsqg_bwd_dkdv_kernel(const dwarf_dsqg_bwd_args a,
-                                                              const float* __restrict__ delta_ws, int tiles, int total) {
-  constexpr int HD = kHeadDim;
-  constexpr int DPL = HD / L;
-  constexpr int KPB = kBlock / L;
-  constexpr int SEG = HD / kPlanes;
-  const dwarf_dsqg_fwd_args& f = a.fwd;
-
-  extern __shared__ float smem[];
-  float* s_se = smem;                               // [J][64]
-  int* s_off = reinterpret_cast<int*>(s_se + f.J * HD);
-
-  const int work = xcd_remap(blockIdx.x, total);
-  const int bhk = work / tiles;
-  const int tile = work - bhk * tiles;
-  const int b = bhk / f.H_kv;
-  const int hk = bhk - b * f.H_kv;
-  const int group = f.H / f.H_kv;
-
-  for (int i = threadIdx.x; i < f.J * HD; i += kBlock) {
-    const int j = i / HD, d = i - j * HD;
-    const float e = f.scale_embed[j * f.se_stride[0] + d * f.se_stride[1]];
-    s_se[i] = f.se_round_bf16 ? round_bf16(e) : e;
-  }
-  for (int j = threadIdx.x; j < f.J; j += kBlock) s_off[j] = f.offsets[j];
-  __syncthreads();
-
-  const int lane = threadIdx.x;
-  const int g = lane % L;
-  const int m = tile * KPB + lane / L;
-  if (m >= f.N) return;  // no barriers below
-  const int wave_m_first = uniform(tile * KPB + (lane / kWave) * (kWave / L));
-  const int wave_m_last = wave_m_first + kWave / L - 1;
-  const int64_t mm = m;
-
-  float kv[DPL], vv[DPL], dk[DPL], dv[DPL];
-  load_f32<T, DPL>(reinterpret_cast<const T*>(f.k) + b * f.k_stride[0] + hk * f.k_stride[1] + mm * f.k_stride[2] + g * DPL, kv);
-  load_f32<T, DPL>(reinterpret_cast<const T*>(f.v) + b * f.v_stride[0] + hk * f.v_stride[1] + mm * f.v_stride[2] + g * DPL, vv);
-#pragma unroll
-  for (int d = 0; d < DPL; ++d) { dk[d] = 0.f; dv[d] = 0.f; }
-  const float4 z4 = *reinterpret_cast<const float4*>(f.z_pre + b * f.z_stride[0] + hk * f.z_stride[1] + mm * f.z_stride[2]);
-  const float zs[4] = {z4.x, z4.y, z4.z, z4.w};
-  float dz[4] = {0.f, 0.f, 0.f, 0.f};
-  constexpr float scale = 0.125f;
-
-  for (int hh = 0; hh < group; ++hh) {
-    const int h = hk * group + hh;
-    const int bh = b * f.H + h;
-    const T* qbase = reinterpret_cast<const T*>(f.q) + b * f.q_stride[0] + h * f.q_stride[1] + g * DPL;
-    const T* dobase = reinterpret_cast<const T*>(a.dout) + b * a.dout_stride[0] + h * a.dout_stride[1] + g * DPL;
-    const float* lsebase = f.lse + b * f.lse_stride[0] + h * f.lse_stride[1];
-    const float* dltbase = delta_ws + static_cast<int64_t>(bh) * f.N;
-    const float* ybase = f.y_pre + b * f.y_stride[0] + h * f.y_stride[1];
-
-    for (int j = 0; j < f.J; ++j) {
-      const int delta = s_off[j];
-      if (wave_m_first + delta >= f.N || wave_m_last + delta < f.query_start) continue;
-      const int n = m + delta;
-      if (n < 0 || n >= f.N) continue;
-      const int64_t nn = n;
-      const float lse = lsebase[nn * f.lse_stride[2]];
-      if (!(lse > -INFINITY)) continue;
-      float qn[DPL], don[DPL];
-      load_f32<T, DPL>(qbase + nn * f.q_stride[2], qn);
-      const float* e = s_se + j * HD + g * DPL;
-      float dot = 0.f;
-#pragma unroll
-      for (int d = 0; d < DPL; ++d) dot = fmaf(qn[d], kv[d] + e[d], dot);
-      dot = group_sum<L>(dot);
-      const float P = dexp<FAST>(fmaf(dot, scale, f.pos_bias[j * f.pb_stride[0] + h * f.pb_stride[1]]) - lse);
-
-      load_f32<T, DPL>(dobase + nn * a.dout_stride[2], don);
-      float gd = 0.f;
-#pragma unroll
-      for (int d = 0; d < DPL; ++d) gd = fmaf(don[d], vv[d], gd);
-      // dV contribution with rotated channels replaced below.
-      float dva[4] = {0.f, 0.f, 0.f, 0.f}, dvb[4] = {0.f, 0.f, 0.f, 0.f};
-      bool far = j >= f.J_small;
-      if (far) {
-        const int i = j - f.J_small;
-        const float4 y4 = *reinterpret_cast<const float4*>(ybase + nn * f.y_stride[2]);
-        const float ys[4] = {y4.x, y4.y, y4.z, y4.w};
-#pragma unroll
-        for (int r = 0; r < kPlanes; ++r) {
-          const int ch = r * SEG + SHIFT;
-          if (ch / DPL != g) continue;
-          const int la = ch % DPL;
-          const float pg = f.phase_gain[i * f.pgain_stride[0] + h * f.pgain_stride[1] + r];
-          const float theta = f.phase_base[i * f.pbase_stride[0] + h * f.pbase_stride[1] + r] + pg * ys[r] * zs[r];
-          float sn, cs;
-          dsincos<FAST>(theta, &sn, &cs);
-          const float va = vv[la], vb = vv[la + 1];
-          const float da = don[la], db = don[la + 1];
-          gd += da * (cs * va - sn * vb - va) + db * (sn * va + cs * vb - vb);
-          const float t = P * (da * (-va * sn - vb * cs) + db * (va * cs - vb * sn));
-          dz[r] = fmaf(t * pg, ys[r], dz[r]);
-          dva[r] = cs * da + sn * db;   // (R^T dO)_a
-          dvb[r] = -sn * da + cs * db;  // (R^T dO)_b
-        }
-      }
-      gd = group_sum<L>(gd);
-      const float dS = P * (gd - dltbase[nn]);
-      const float cds = scale * dS;
-#pragma unroll
-      for (int d = 0; d < DPL; ++d) {
-        dk[d] = fmaf(cds, qn[d], dk[d]);
-        dv[d] = fmaf(P, don[d], dv[d]);
-      }
-      if (far) {
-#pragma unroll
-        for (int r = 0; r < kPlanes; ++r) {
-          const int ch = r * SEG + SHIFT;
-          if (ch / DPL != g) continue;
-          const int la = ch % DPL;
-          dv[la] = fmaf(P, dva[r] - don[la], dv[la]);
-          dv[la + 1] = fmaf(P, dvb[r] - don[la + 1], dv[la + 1]);
-        }
-      }
-    }
-  }
-
-  store_from_f32<T, DPL>(reinterpret_cast<T*>(a.dk) + b * a.dk_stride[0] + hk * a.dk_stride[1] + mm * a.dk_stride[2] + g * DPL, dk);
-  store_from_f32<T, DPL>(reinterpret_cast<T*>(a.dv) + b * a.dv_stride[0] + hk * a.dv_stride[1] + mm * a.dv_stride[2] + g * DPL, dv);
-  float dzo[4];
-#pragma unroll
-  for (int r = 0; r < kPlanes; ++r) dzo[r] = group_sum<L>(dz[r]);
-  if (g == 0)
-    *reinterpret_cast<float4*>(a.dz_pre + (static_cast<int64_t>(bhk) * f.N + m) * kPlanes) =
-        make_float4(dzo[0], dzo[1], dzo[2], dzo[3]);
-}
 
 // ---- bf16 dK/dV launch: four lanes per key ------------------------------
 // A workgroup of 4 waves owns 64 consecutive keys of one (b, kv head); wave w
@@ -775,38 +643,12 @@ RedPlan make_red_plan(const dwarf_dsqg_bwd_args& a, const BwdWorkspace& ws) {
   return p;
 }
 
-template <typename T, int L, bool FAST>
-hipError_t launch_dkdv_typed(const dwarf_dsqg_bwd_args& a, const BwdWorkspace& ws, hipStream_t stream) {
-  const dwarf_dsqg_fwd_args& f = a.fwd;
-  constexpr int KPB = kBlock / L;
-  const float* delta = reinterpret_cast<const float*>(static_cast<char*>(a.workspace) + ws.delta_off);
-  const int tiles = (f.N + KPB - 1) / KPB;
-  const int total_k = tiles * f.B * f.H_kv;
-  const size_t lds_k = static_cast<size_t>(f.J) * (kHeadDim + 1) * sizeof(float);
-#define DWARF_DKDV_CASE(S)                                                                                    \
-  case S:                                                                                                     \
-    hipLaunchKernelGGL((dsqg_bwd_dkdv_kernel<T, S, L, FAST>), dim3(total_k), dim3(kBlock), lds_k, stream, a, \
-                       delta, tiles, total_k);                                                                \
-    break;
-  switch (f.plane_shift) {
-    DWARF_DKDV_CASE(0) DWARF_DKDV_CASE(1) DWARF_DKDV_CASE(2) DWARF_DKDV_CASE(3) DWARF_DKDV_CASE(4)
-    DWARF_DKDV_CASE(5) DWARF_DKDV_CASE(6) DWARF_DKDV_CASE(7) DWARF_DKDV_CASE(8) DWARF_DKDV_CASE(9)
-    DWARF_DKDV_CASE(10) DWARF_DKDV_CASE(11) DWARF_DKDV_CASE(12) DWARF_DKDV_CASE(13) DWARF_DKDV_CASE(14)
-    default:
-      return hipErrorInvalidValue;
-  }
-#undef DWARF_DKDV_CASE
-  return hipGetLastError();
-}
-
-constexpr int kLanesBwd = 2;
-
 }  // namespace
 
 BwdWorkspace bwd_workspace_layout(const dwarf_dsqg_bwd_args& a) {
   const dwarf_dsqg_fwd_args& f = a.fwd;
   BwdWorkspace w{};
-  const int kTile = dq_tile_queries(f.dtype);
+  const int kTile = dq_tile_queries();
   w.dq_tiles = (f.N + kTile - 1) / kTile;
   const int total_tiles = w.dq_tiles * f.B * f.H;
   const int JL = f.J_large > 0 ? f.J_large : 1;
@@ -814,8 +656,6 @@ BwdWorkspace bwd_workspace_layout(const dwarf_dsqg_bwd_args& a) {
     // Persistent workgroups, all resident: the gather launch (dQ, dY, dS,
     // dPhase partials per tile) and the dSE launch, whose workgroups
     // accumulate dSE in their own slots (dPB partials per tile).
-    w.dq_tpw = 0;
-    w.dq_ntg = 0;
     // beside a concurrent dK/dV launch (the delta stage) the dQ launch takes 400 workgroups (50 per XCD,
     // about three per two CUs) and leaves the rest to dK/dV, so that the two streams end together: at
     // B15 H8 T2048 the step measured 0.550-0.552 ms with 400 workgroups, 0.556 with 384 and 0.572 with 512
@@ -828,23 +668,17 @@ BwdWorkspace bwd_workspace_layout(const dwarf_dsqg_bwd_args& a) {
     w.pb_rows = f.B * w.dq_tiles;
     w.ph_rows = f.B * w.dq_tiles;
   } else {
-    // Two 4-wave workgroups fit per CU: size the tile groups so every
-    // workgroup is resident at once (at most 512 on 256 CUs).
-    w.dq_tpw = (total_tiles + 511) / 512;
-    if (w.dq_tpw < 1) w.dq_tpw = 1;
-    if (w.dq_tpw > 16) w.dq_tpw = 16;
-    if (w.dq_tpw > w.dq_tiles) w.dq_tpw = w.dq_tiles > 0 ? w.dq_tiles : 1;
-    w.dq_ntg = (w.dq_tiles + w.dq_tpw - 1) / w.dq_tpw;
-    w.dq_wgs = f.B * f.H * w.dq_ntg;
-    w.pb_rows = f.B * w.dq_ntg;
-    w.ph_rows = 4 * f.B * w.dq_ntg;   // one row per wave
+    const F32Plan p = f32_plan(f);
+    w.dq_wgs = f.B * f.H * p.se_ntg;
+    w.pb_rows = f.B * p.se_ntg;
+    w.ph_rows = f.B * p.dq_ntg;
   }
   w.red_groups_se = (w.dq_wgs + kRedRows - 1) / kRedRows;
   w.red_groups_pb = (w.pb_rows + kRedRows - 1) / kRedRows;
   w.red_groups_ph = (w.ph_rows + kRedRows - 1) / kRedRows;
   size_t off = 0;
-  w.delta_off = off;   // bf16: (delta, log2 lse) pairs; fp32: delta
-  w.delta_bytes = static_cast<size_t>(f.B) * f.H * f.N * 2 * sizeof(float);
+  w.delta_off = off;   // (delta, log2 lse) pairs
+  w.delta_bytes = f.dtype == DWARF_BF16 ? static_cast<size_t>(f.B) * f.H * f.N * 2 * sizeof(float) : 0;
   off += align256(w.delta_bytes);
   w.part_se_off = off;
   w.part_se_bytes = static_cast<size_t>(w.dq_wgs) * f.J * kHeadDim * sizeof(float);
@@ -856,7 +690,7 @@ BwdWorkspace bwd_workspace_layout(const dwarf_dsqg_bwd_args& a) {
   w.part_ph_bytes = static_cast<size_t>(f.H) * w.ph_rows * JL * 8 * sizeof(float);
   off += align256(w.part_ph_bytes);
   w.ds_off = off;
-  w.ds_bytes = f.dtype == DWARF_BF16 ? static_cast<size_t>(f.B) * f.H * f.J * f.N * sizeof(float) : 0;
+  w.ds_bytes = static_cast<size_t>(f.B) * f.H * f.J * (f.dtype == DWARF_BF16 ? f.N : 2 * f32_plan(f).np) * sizeof(float);
   off += align256(w.ds_bytes);
   w.red_off = off;
   w.red_bytes = (static_cast<size_t>(w.red_groups_se) * f.J * kHeadDim +
@@ -903,7 +737,7 @@ hipError_t launch_dsqg_bwd(const dwarf_dsqg_bwd_args& a, const BwdWorkspace& ws,
   }
   if (do_dkdv) {
     if (a.fwd.dtype == DWARF_BF16) return launch_dkdv_bf16_k4(a, ws, stream);
-    return launch_dkdv_typed<float, kLanesBwd, false>(a, ws, stream);
+    return launch_f32_dkdv(a, ws, stream);
   }
   return hipSuccess;
 }

@@ -476,3 +476,58 @@ def test_lattice_without_far_offsets(pkg, device, dtype):
         assert max_abs(out, ro) < BF16_ABS
         for n in used:
             assert max_abs(grads[n], rg[n]) < BF16_ABS, (n, max_abs(grads[n], rg[n]))
+
+
+@pytest.mark.parametrize("B,H,Hkv,N,shift,near,far,online", [
+    (1, 1, 1, 17, 3, 17, 0, True),          # a second tile of one row; a pair across two lanes; no far offsets
+    (2, 2, 1, 16, 7, 0, 5, True),           # one whole tile; no near offsets; shorter than most offsets
+    (1, 6, 2, 131, 11, 17, 30, False),      # a group of three heads, the offline softmax
+    (1, 2, 2, 300, 14, 17, 133, True),      # 150 offsets (four 16-offset blocks to a wave)
+    (3, 8, 8, 1040, 4, 6, 23, True),        # several tiles to a workgroup
+    (1, 3, 3, 2, 1, 2, 0, True),            # two rows
+])
+def test_fp32_kernels_edges(pkg, device, B, H, Hkv, N, shift, near, far, online):
+    """The fp32 launches where their tiles, lists and lane pairs end, against the float64 oracle at the fp32 bar.
+    Sums of at most a few thousand terms; dpos_bias and the phase gradients of a few rows cancel to little, so the
+    bar there is 1e-5 of the sum of magnitudes' scale, taken as the largest gradient of the table."""
+    full = lattice(pkg)
+    extra = [48 + 3 * i for i in range(200) if 48 + 3 * i not in full]
+    offsets = full[:near] + sorted((full[17:] + extra)[:far])
+    x = make_inputs(B, H, Hkv, N, offsets, near, seed=400 + N, dtype=torch.float32, plane_shift=shift, gain_std=6.0)
+    dout = torch.randn(B, H, N, 64, generator=torch.Generator().manual_seed(N))
+    qs = min(2, N) if N > 16 else 1
+    out, grads = gpu_fwd_bwd(pkg, x, offsets, near, shift, qs, dout, device, online=online)
+    ro, _, rg = oracle_fwd_bwd(x, offsets, near, shift, qs, dout, round_se=False)
+    assert max_abs(out, ro) <= FP32_REL * float(ro.abs().max().clamp_min(1.0))
+    for n in NAMES:
+        ref = torch.zeros_like(grads[n]).double().cpu() if rg[n] is None else rg[n]   # None: no far offset takes part
+        assert max_abs(grads[n], ref) <= FP32_REL * float(ref.abs().max().clamp_min(1e-3)), n
+
+
+def test_fp32_masked_offsets_and_foreign_nan(pkg, device):
+    """pos_bias of -inf takes an offset out (as an offset list without it gives, also where every source of a row
+    is masked: zeros), and NaN in a key, value or z row reaches only the queries that have it as a source and the
+    gradients formed from them."""
+    offsets, js, N = [1, 2, 5, 48, 64, 130], 3, 200
+    x = make_inputs(1, 2, 2, N, offsets, js, seed=7, dtype=torch.float32, plane_shift=3)
+    dout = torch.randn(1, 2, N, 64, generator=torch.Generator().manual_seed(8))
+    x["pos_bias"][[0, 3]] = float("-inf")
+    out, grads = gpu_fwd_bwd(pkg, x, offsets, js, 3, 1, dout, device)
+    keep = [1, 2, 4, 5]
+    y = {n: (t[keep] if n in ("pos_bias", "scale_embed") else t[[1, 2]] if n.startswith("phase") else t) for n, t in x.items()}
+    ro, _, rg = oracle_fwd_bwd(y, [offsets[i] for i in keep], 2, 3, 1, dout, round_se=False)
+    assert rel_err(out, ro) < FP32_REL and not out[:, :, 1].any()
+    for n in ("q", "k", "v", "y_pre", "z_pre"):
+        assert rel_err(grads[n], rg[n]) < FP32_REL, n
+    bad = 77
+    z = {n: t.clone() for n, t in x.items()}
+    for n in ("k", "v", "z_pre"):
+        z[n][:, :, bad] = float("nan")
+    o2, g2 = gpu_fwd_bwd(pkg, z, offsets, js, 3, 1, dout, device)
+    hit = torch.zeros(N, dtype=torch.bool)
+    for d in offsets:   # a masked offset's NaN score is NaN too
+        if bad + d < N:
+            hit[bad + d] = True
+    assert torch.equal(o2[:, :, ~hit], out[:, :, ~hit])
+    assert torch.isnan(o2[:, :, hit]).any(-1).all()
+    assert torch.equal(g2["q"][:, :, ~hit], grads["q"][:, :, ~hit])
