@@ -282,7 +282,18 @@ class PacketBwdArgs(ctypes.Structure):
 
 # ---- include/dwarf_block.h ----
 BLOCK_SYMBOLS = ("dwarf_normalize_probes", "dwarf_dsqg_bwd_two_streams", "dwarf_head_gate_fwd",
-                 "dwarf_head_gate_bwd_workspace_bytes", "dwarf_head_gate_bwd")
+                 "dwarf_head_gate_bwd_workspace_bytes", "dwarf_head_gate_bwd",
+                 "dwarf_linear_wgrad_workspace_bytes", "dwarf_linear_wgrad")
+
+
+class LinearWgradArgs(ctypes.Structure):
+    _fields_ = [
+        ("M", c_int64), ("O", c_int32), ("I", c_int32),
+        ("dy", c_void_p), ("dy_stride", c_int64),
+        ("x", c_void_p), ("x_stride", c_int64),
+        ("dw", c_void_p), ("db", c_void_p),
+        ("workspace", c_void_p), ("workspace_bytes", c_size_t),
+    ]
 
 
 class HeadGateFwdArgs(ctypes.Structure):
@@ -401,6 +412,10 @@ def load() -> ctypes.CDLL:
     lib.dwarf_normalize_probes.argtypes = [c_void_p, c_void_p, c_void_p, c_void_p]
     lib.dwarf_dsqg_bwd_two_streams.restype = c_int
     lib.dwarf_dsqg_bwd_two_streams.argtypes = [POINTER(DsqgBwdArgs), c_int32, c_void_p, c_void_p]
+    lib.dwarf_linear_wgrad_workspace_bytes.restype = c_size_t
+    lib.dwarf_linear_wgrad_workspace_bytes.argtypes = [POINTER(LinearWgradArgs)]
+    lib.dwarf_linear_wgrad.restype = c_int
+    lib.dwarf_linear_wgrad.argtypes = [POINTER(LinearWgradArgs), c_void_p]
     lib.dwarf_head_gate_fwd.restype = c_int
     lib.dwarf_head_gate_fwd.argtypes = [POINTER(HeadGateFwdArgs), c_void_p]
     lib.dwarf_head_gate_bwd_workspace_bytes.restype = c_size_t

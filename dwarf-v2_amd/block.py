@@ -22,12 +22,14 @@ verify_mode, max_group_spread_observed, plane_shift, backend,
 online_softmax, if_gain, out_proj, dropout.
 
 Under bf16 autocast, without kv_inject and without support cropping (the
-trainer's blocks), everything between the two projections is one autograd
-Function on the fused projection [B, N, 4D] (``_DSQGBlockFn``): the attention
-reads q, k and v as views of it, the per-head gain and the content gate are
-one launch after it (csrc/block.hip), and the backward writes dq, dk, dv and
-the gate's gradient straight into one [B, N, 4D] gradient.  Each product is
-rounded where the unfused expression rounds it.
+trainer's blocks), the whole block is one autograd Function
+(``_DSQGBlockFn``): the attention reads q, k and v as views of the fused
+projection [B, N, 4D], the per-head gain and the content gate are one launch
+after it (csrc/block.hip), the backward writes dq, dk, dv and the gate's
+gradient straight into one [B, N, 4D] gradient, and the projections' weight
+gradients are split over the tokens (csrc/wgrad.hip).  Each product is
+rounded where the unfused expression rounds it, except that the weight
+gradients stay fp32.
 """
 
 from __future__ import annotations
@@ -112,6 +114,25 @@ def head_gate_backward(dgated, out, gain, gate, dgate, *, lse=None, query_start=
     return dout, dgain
 
 
+def linear_wgrad(dy: torch.Tensor, x: torch.Tensor, bias: bool) -> tuple[torch.Tensor, torch.Tensor | None]:
+    """Raw launch: (dW [O,I], db [O] or None) fp32 of y = x W^T + b from dy [..., O] and x [..., I] bf16."""
+    dy, x = (t.reshape(-1, t.shape[-1]) for t in (dy, x))
+    dy, x = (t if _rows_ok(t) and t.stride(0) >= t.shape[1] else t.clone(memory_format=torch.contiguous_format)
+             for t in (dy, x))
+    lib = _lib.load()
+    dw = torch.empty((dy.shape[1], x.shape[1]), device=dy.device, dtype=torch.float32)
+    db = torch.empty(dy.shape[1], device=dy.device, dtype=torch.float32) if bias else None
+    a = _lib.LinearWgradArgs()
+    a.M, a.O, a.I = dy.shape[0], dy.shape[1], x.shape[1]
+    a.dy, a.dy_stride, a.x, a.x_stride = dy.data_ptr(), dy.stride(0), x.data_ptr(), x.stride(0)
+    a.dw, a.db = dw.data_ptr(), None if db is None else db.data_ptr()
+    ws = torch.empty(max(int(lib.dwarf_linear_wgrad_workspace_bytes(ctypes.byref(a))), 16), device=dy.device,
+                     dtype=torch.uint8)
+    a.workspace, a.workspace_bytes = ws.data_ptr(), ws.numel()
+    _lib.check(lib.dwarf_linear_wgrad(ctypes.byref(a), _stream(dy.device)), "dwarf_linear_wgrad")
+    return dw, db
+
+
 def block_forward(qkvg, pos_bias, scale_embed, phase_base, phase_gain, query_probes, key_probes, gain, offsets, heads,
                   j_small, j_large, plane_shift, query_start, schedule):
     """Raw launches from the fused projection [B,N,4D] (bf16, contiguous) to the gated heads [B,N,D]: returns
@@ -158,61 +179,86 @@ def block_backward(dgated, qkvg, pos_bias, scale_embed, phase_base, phase_gain, 
 
 
 class _DSQGBlockFn(torch.autograd.Function):
-    """The block between its projections as one node: gated heads from the fused projection, over the custom
-    ops ``torch.ops.dwarf.dsqg_block_fwd`` / ``dsqg_block_bwd`` (registered in ``ops.py``).  Probes: normalised
-    fp32 [4,64], without gradient."""
+    """The block from its input to its output projection as one node (bf16): the two projections, and between them
+    the custom ops ``torch.ops.dwarf.dsqg_block_fwd`` / ``dsqg_block_bwd``; the projections' weight and bias
+    gradients come from ``torch.ops.dwarf.linear_wgrad`` (all registered in ``ops.py``) in fp32.  Probes:
+    normalised fp32 [4,64], without gradient; a projection's bias may be None."""
 
     @staticmethod
-    def forward(ctx, qkvg, pos_bias, scale_embed, phase_base, phase_gain, gain, query_probes, key_probes, offsets_dev,
-                heads, j_small, j_large, plane_shift, query_start, schedule, bwd_schedule):
+    def forward(ctx, x, w_in, b_in, w_out, b_out, pos_bias, scale_embed, phase_base, phase_gain, gain, query_probes,
+                key_probes, offsets_dev, heads, j_small, j_large, plane_shift, query_start, schedule, bwd_schedule):
         args = (int(heads), int(j_small), int(j_large), int(plane_shift), int(query_start))
         ctx.args = (*args, int(bwd_schedule))
+        bf16 = torch.bfloat16
+        x16, wi, wo = x.to(bf16), w_in.to(bf16), w_out.to(bf16)
+        qkvg = F.linear(x16, wi, None if b_in is None else b_in.to(bf16))
         gated, out, lse, y, z = torch.ops.dwarf.dsqg_block_fwd(qkvg, pos_bias, scale_embed, phase_base, phase_gain,
                                                                query_probes, key_probes, gain, offsets_dev, *args,
                                                                int(schedule))
-        ctx.save_for_backward(qkvg, pos_bias, scale_embed, phase_base, phase_gain, gain, query_probes, key_probes,
-                              offsets_dev, out, lse, y, z)
-        return gated
+        result = F.linear(gated, wo, None if b_out is None else b_out.to(bf16))
+        ctx.save_for_backward(x16, wi, wo, qkvg, gated, pos_bias, scale_embed, phase_base, phase_gain, gain,
+                              query_probes, key_probes, offsets_dev, out, lse, y, z)
+        ctx.dtypes = tuple(None if t is None else t.dtype for t in (x, w_in, b_in, w_out, b_out))
+        return result
 
     @staticmethod
-    def backward(ctx, dgated):
-        qkvg, pb, se, pbase, pgain, gain, qp, kp, offsets, out, lse, y, z = ctx.saved_tensors
-        g = torch.ops.dwarf.dsqg_block_bwd(dgated, qkvg, pb, se, pbase, pgain, qp, kp, gain, offsets, out, lse, y, z,
-                                           *ctx.args)
+    def backward(ctx, dy):
+        x16, wi, wo, qkvg, gated, pb, se, pbase, pgain, gain, qp, kp, offsets, out, lse, y, z = ctx.saved_tensors
+        dt_x, dt_wi, dt_bi, dt_wo, dt_bo = ctx.dtypes
+        need = ctx.needs_input_grad
+        dy = dy.to(torch.bfloat16)
+
+        def weights(grad, inp, dt_w, dt_b, need_w, need_b):
+            if not (need_w or need_b):
+                return None, None
+            dw, db = torch.ops.dwarf.linear_wgrad(grad, inp, dt_b is not None)
+            return dw.to(dt_w), None if dt_b is None else db.to(dt_b)
+
+        dwo, dbo = weights(dy, gated, dt_wo, dt_bo, need[3], need[4])
+        g = torch.ops.dwarf.dsqg_block_bwd(torch.matmul(dy, wo), qkvg, pb, se, pbase, pgain, qp, kp, gain, offsets, out,
+                                           lse, y, z, *ctx.args)
         dqkvg, dpb, dse, dpbase, dpgain, dgain = g
-        return (dqkvg, dpb, dse, dpbase, dpgain, dgain.reshape(gain.shape)) + (None,) * 10
+        dwi, dbi = weights(dqkvg, x16, dt_wi, dt_bi, need[1], need[2])
+        dx = torch.matmul(dqkvg, wi).to(dt_x) if need[0] else None
+        return (dx, dwi, dbi, dwo, dbo, dpb, dse, dpbase, dpgain, dgain.reshape(gain.shape)) + (None,) * 10
 
 
 def _plain_linear(m) -> bool:
-    """An nn.Linear nothing hooks into: it takes the bf16 product where autocast would have cast an fp32 one."""
-    return (type(m) is torch.nn.Linear and not m._forward_pre_hooks and not m._forward_hooks
+    """An nn.Linear nothing hooks into, of whole 16-byte rows: its forward is F.linear on its weight and bias."""
+    return (type(m) is torch.nn.Linear and m.in_features % 8 == 0 and m.out_features % 8 == 0
+            and not m._forward_pre_hooks and not m._forward_hooks
             and not m._backward_hooks and not m._backward_pre_hooks)
 
 
-def _one_node(block, proj: torch.Tensor) -> bool:
-    """Whether the block between its projections runs as ``_DSQGBlockFn``: bf16 autocast (so that the output
-    projection reads bf16 either way), frozen phase probes, the fp32 gain of the module."""
-    if not (proj.is_cuda and proj.dtype == torch.bfloat16 and torch.is_autocast_enabled("cuda")
-            and torch.get_autocast_dtype("cuda") == torch.bfloat16):
+def _one_node(block, x: torch.Tensor) -> bool:
+    """Whether the block runs as ``_DSQGBlockFn``: bf16 autocast (both projections read and write bf16), plain
+    linear projections, frozen phase probes, the fp32 gain of the module."""
+    if not (x.is_cuda and torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") == torch.bfloat16):
         return False
     if torch.is_grad_enabled() and (block.query_probes.requires_grad or block.key_probes.requires_grad):
         return False
-    return (block.head_dim == HEAD_DIM and proj.shape[-1] == 4 * block.num_heads * HEAD_DIM
+    proj, out, D = block.qkvg_proj, block.out_proj, block.num_heads * HEAD_DIM
+    return (_plain_linear(proj) and _plain_linear(out) and block.head_dim == HEAD_DIM
+            and proj.in_features == x.shape[-1] == D and proj.out_features == 4 * D and out.in_features == D
+            and proj.weight.device == x.device and out.weight.device == x.device
             and block.if_gain.dtype == torch.float32 and block.if_gain.numel() == block.num_heads
-            and str(block.backend).lower() in ("auto", "triton", "hip") and _plain_linear(block.out_proj))
+            and str(block.backend).lower() in ("auto", "triton", "hip"))
 
 
-def _gated_heads(block, proj: torch.Tensor, query_start: int) -> torch.Tensor:
-    H = block.num_heads
-    q, k, v, _ = proj.split(proj.shape[-1] // 4, dim=-1)
-    q, k, v = (_heads(t, H) for t in (q, k, v))
-    _check_call(q, k, v, None, None, block.j_val, block.j_small, block.j_large, block.offsets_dev, block.grouped_mode_id)
-    qp, kp = normalized_probe_banks(block.query_probes, block.key_probes, proj.device)
+def _block_node(block, x: torch.Tensor, query_start: int) -> torch.Tensor:
+    H, N = block.num_heads, x.shape[1]
+    # the op's own checks, on the shapes its q, k and v views will have
+    probe = torch.empty(1, device=x.device, dtype=torch.bfloat16).expand(x.shape[0], H, N, HEAD_DIM)
+    _check_call(probe, probe, probe, None, None, block.j_val, block.j_small, block.j_large, block.offsets_dev,
+                block.grouped_mode_id)
+    qp, kp = normalized_probe_banks(block.query_probes, block.key_probes, x.device)
     phase_gate = torch.sigmoid(block.phase_gate)[:, None, None]
+    proj, out = block.qkvg_proj, block.out_proj
     return _DSQGBlockFn.apply(
-        proj, block.pos_bias.float(), block.centered_scale_embed.float(), (block.phase_base * phase_gate).float(),
-        (block.phase_gain * phase_gate).float(), block.if_gain.reshape(-1), qp, kp, block.offsets_dev, H,
-        int(block.j_small), int(block.j_large), int(block.plane_shift), max(0, min(int(query_start), proj.shape[1])),
+        x, proj.weight, proj.bias, out.weight, out.bias, block.pos_bias.float(), block.centered_scale_embed.float(),
+        (block.phase_base * phase_gate).float(), (block.phase_gain * phase_gate).float(), block.if_gain.reshape(-1), qp,
+        kp, block.offsets_dev, H, int(block.j_small), int(block.j_large), int(block.plane_shift),
+        max(0, min(int(query_start), N)),
         *(schedule_for(block.grouped_mode_id, bool(block.online_softmax), int(block.j_small), back)
           for back in (False, True)))
 
@@ -253,11 +299,10 @@ def dsqg_block_forward(block, x: torch.Tensor, kv_inject=None) -> torch.Tensor:
     key_end = max(0, N - query_start)
     if block.support_crop_projections and query_start >= block.support_crop_min_offset:
         q, k, v, gate = _cropped_projections(block, x, query_start, key_end)
+    elif kv_inject is None and _one_node(block, x):
+        return block.dropout(_block_node(block, x, query_start))
     else:
-        proj = block.qkvg_proj(x)
-        if kv_inject is None and _one_node(block, proj):
-            return block.dropout(block.out_proj(_gated_heads(block, proj, query_start)))
-        q, k, v, gate = proj.split(D, dim=-1)
+        q, k, v, gate = block.qkvg_proj(x).split(D, dim=-1)
     # [B, N, H*hd] -> [B, H, N, hd] views over the projection rows
     q, k, v = (t.reshape(B, N, H, hd).permute(0, 2, 1, 3) for t in (q, k, v))
     if kv_inject is not None:

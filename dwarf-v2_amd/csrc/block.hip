@@ -118,6 +118,7 @@ __global__ __launch_bounds__(kBlock) void head_gate_gain_kernel(const float* __r
                                                                 unsigned H, float* __restrict__ dgain) {
   __shared__ float s_sum[kBlock / kWave];
   float x = 0.f;
+#pragma unroll 8
   for (unsigned i = blockIdx.x + threadIdx.x * H; i < slots; i += kBlock * H) x += part[i];
   x = wave_sum_to_last(x);
   if (threadIdx.x % kWave == kWave - 1) s_sum[threadIdx.x / kWave] = x;

@@ -44,6 +44,8 @@ hipError_t launch_interference_packet_fwd(const dwarf_packet_fwd_args& a, hipStr
 hipError_t launch_interference_packet_bwd(const dwarf_packet_bwd_args& a, hipStream_t stream);
 hipError_t launch_phase_probe_fwd(const dwarf_phase_probe_fwd_args& a, hipStream_t stream);
 hipError_t launch_phase_probe_bwd(const dwarf_phase_probe_bwd_args& a, hipStream_t stream);
+size_t linear_wgrad_workspace(const dwarf_linear_wgrad_args& a);
+hipError_t launch_linear_wgrad(const dwarf_linear_wgrad_args& a, hipStream_t stream);
 hipError_t launch_normalize_probes(const float* q, const float* k, float* out, hipStream_t stream);
 size_t head_gate_bwd_workspace(const dwarf_head_gate_bwd_args& a);
 hipError_t launch_head_gate_fwd(const dwarf_head_gate_fwd_args& a, hipStream_t stream);
@@ -763,6 +765,34 @@ int dwarf_dsqg_bwd_two_streams(const dwarf_dsqg_bwd_args* args, int32_t pairs_re
   if (fork) (void)hipEventDestroy(fork);
   if (join) (void)hipEventDestroy(join);
   return rc;
+}
+
+size_t dwarf_linear_wgrad_workspace_bytes(const dwarf_linear_wgrad_args* a) {
+  return a && a->M > 0 && a->O > 0 && a->I > 0 ? dwarf::linear_wgrad_workspace(*a) : 0;
+}
+
+int dwarf_linear_wgrad(const dwarf_linear_wgrad_args* args, dwarf_stream_t stream) {
+  if (!args) return fail(DWARF_ERR_INVALID_ARGUMENT, "args is NULL");
+  const dwarf_linear_wgrad_args& a = *args;
+  if (a.M < 0 || a.O <= 0 || a.I <= 0) return fail(DWARF_ERR_INVALID_ARGUMENT, "bad sizes O=%d I=%d", a.O, a.I);
+  if (!a.dw || !aligned16(a.dw) || (a.db && !aligned16(a.db)))
+    return fail(DWARF_ERR_INVALID_ARGUMENT, "dw and db must be 16-byte aligned");
+  if (a.O % 8 || a.I % 8) return fail(DWARF_ERR_UNSUPPORTED, "O=%d and I=%d must be multiples of 8", a.O, a.I);
+  const hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  if (a.M == 0) {   // sums over nothing
+    int rc = zero_floats(a.dw, static_cast<int64_t>(a.O) * a.I, s, "dwarf_linear_wgrad");
+    return rc || !a.db ? rc : zero_floats(a.db, a.O, s, "dwarf_linear_wgrad");
+  }
+  const int64_t sy[2] = {a.dy_stride, 1}, sx[2] = {a.x_stride, 1};
+  int rc;
+  if ((rc = check_rows("dy", a.dy, sy, 1, DWARF_BF16))) return rc;
+  if ((rc = check_rows("x", a.x, sx, 1, DWARF_BF16))) return rc;
+  if (a.dy_stride < a.O || a.x_stride < a.I || a.dy_stride > (1 << 22) || a.x_stride > (1 << 22))
+    return fail(DWARF_ERR_UNSUPPORTED, "row strides must lie between the row length and 2^22 elements");
+  const size_t need = dwarf::linear_wgrad_workspace(a);
+  if (!a.workspace || a.workspace_bytes < need || !aligned16(a.workspace))
+    return fail(DWARF_ERR_WORKSPACE, "workspace needs %zu bytes, 16-byte aligned, got %zu", need, a.workspace_bytes);
+  return hip_status(dwarf::launch_linear_wgrad(a, s), "dwarf_linear_wgrad");
 }
 
 static int check_gate(const dwarf_head_gate_fwd_args& a) {

@@ -6,7 +6,7 @@
 ``dwarf::npci_fwd``, ``dwarf::npci_bwd``, ``dwarf::packet_pool_fwd``,
 ``dwarf::packet_pool_bwd``, ``dwarf::packet_fwd``, ``dwarf::packet_bwd``,
 ``dwarf::normalize_probes``,
-``dwarf::dsqg_block_fwd`` and ``dwarf::dsqg_block_bwd`` are
+``dwarf::linear_wgrad``, ``dwarf::dsqg_block_fwd`` and ``dwarf::dsqg_block_bwd`` are
 custom ops with fake (shape-only) implementations, so ``torch.compile`` traces
 the DSQG, EMA, phase-probe, NPCI and InterferencePacket autograd Functions
 without graph breaks (the trainer
@@ -135,6 +135,20 @@ def _normalize_probes_fake(query_probes, key_probes):
 
 
 # ---- the DSQG block between its projections ---------------------------------------------------
+@torch.library.custom_op("dwarf::linear_wgrad", mutates_args=())
+def linear_wgrad(dy: Tensor, x: Tensor, bias: bool) -> tuple[Tensor, Tensor]:
+    """(dW [O,I], db [O]; empty [0] without a bias) fp32 of y = x W^T + b, from dy [...,O] and x [...,I] bf16."""
+    dw, db = _block.linear_wgrad(dy, x, bias)
+    return dw, db if db is not None else dw.new_empty((0,))
+
+
+@linear_wgrad.register_fake
+def _linear_wgrad_fake(dy, x, bias):
+    f32 = torch.float32
+    return (dy.new_empty((dy.shape[-1], x.shape[-1]), dtype=f32),
+            dy.new_empty((dy.shape[-1] if bias else 0,), dtype=f32))
+
+
 @torch.library.custom_op("dwarf::dsqg_block_fwd", mutates_args=())
 def dsqg_block_fwd(qkvg: Tensor, pos_bias: Tensor, scale_embed: Tensor, phase_base: Tensor, phase_gain: Tensor,
                    query_probes: Tensor, key_probes: Tensor, gain: Tensor, offsets: Tensor, heads: int, j_small: int,

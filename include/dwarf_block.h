@@ -1,8 +1,8 @@
 /*
  * Entry points for the DSQG block around the attention op (libdwarf_dsqg.so,
  * gfx950): the normalised phase probes, the backward's two streams in one
- * call, and the per-head gain and content gate after the attention, forward
- * and backward.  Conventions (status codes, strides in elements, dwarf_stream_t)
+ * call, the per-head gain and content gate after the attention, forward and
+ * backward, and the projections' weight gradients.  Conventions (status codes, strides in elements, dwarf_stream_t)
  * are those of dwarf_dsqg.h.
  */
 #ifndef DWARF_BLOCK_H
@@ -28,6 +28,25 @@ int dwarf_normalize_probes(const float* query_probes, const float* key_probes, f
  */
 int dwarf_dsqg_bwd_two_streams(const dwarf_dsqg_bwd_args* args, int32_t pairs_ready, dwarf_stream_t stream,
                                dwarf_stream_t side);
+
+/*
+ * The weight and bias gradients of y = x W^T + b over M rows: dw[o][i] = sum_m dy[m][o] x[m][i] and
+ * db[o] = sum_m dy[m][o], fp32 sums in a fixed order.  dy [M,O] and x [M,I] bf16, unit column stride, row strides
+ * in elements; O, I and the strides multiples of 8, rows 16-byte aligned; dw [O,I] and db [O] (may be NULL) fp32,
+ * contiguous, 16-byte aligned.
+ */
+typedef struct {
+  int64_t M;
+  int32_t O, I;
+  const void* dy; int64_t dy_stride;
+  const void* x; int64_t x_stride;
+  float* dw;
+  float* db;
+  void* workspace; size_t workspace_bytes;   /* 16-byte aligned */
+} dwarf_linear_wgrad_args;
+
+size_t dwarf_linear_wgrad_workspace_bytes(const dwarf_linear_wgrad_args* args);
+int dwarf_linear_wgrad(const dwarf_linear_wgrad_args* args, dwarf_stream_t stream);
 
 /*
  * gated[b,n,h*64+d] = bf16((out[b,h,n,d] * gain[h]) * bf16(sigmoid(gate[b,n,h*64+d]))), the products in

@@ -312,7 +312,8 @@ def test_unknown_schedule_bits_refused_without_gpu(pkg, lib):
 
 
 BLOCK_HEADER = os.path.join(ROOT, "include", "dwarf_block.h")
-BLOCK_STRUCTS = {"dwarf_head_gate_fwd_args": "HeadGateFwdArgs", "dwarf_head_gate_bwd_args": "HeadGateBwdArgs"}
+BLOCK_STRUCTS = {"dwarf_head_gate_fwd_args": "HeadGateFwdArgs", "dwarf_head_gate_bwd_args": "HeadGateBwdArgs",
+                 "dwarf_linear_wgrad_args": "LinearWgradArgs"}
 
 
 def test_block_header_exports_and_layout(pkg, lib, tmp_path):
@@ -361,3 +362,14 @@ def test_block_entries_refuse_bad_calls_without_gpu(pkg, lib):
     f.gate = 0x10002
     assert lib.dwarf_head_gate_fwd(ctypes.byref(f), None) == bad
     assert b"16-byte" in lib.dwarf_last_error()
+    w = L.LinearWgradArgs()
+    w.M, w.O, w.I, w.dy, w.x, w.dw, w.db = 30720, 2048, 512, 0x10000, 0x10000, 0x10000, 0x10000
+    w.dy_stride, w.x_stride = 2048, 512
+    # 32 output tiles: 8 splits of 60 steps, partial dW and db
+    assert lib.dwarf_linear_wgrad_workspace_bytes(ctypes.byref(w)) == 8 * (2048 * 512 + 2048) * 4
+    assert lib.dwarf_linear_wgrad(ctypes.byref(w), None) == L.DWARF_ERR_WORKSPACE
+    w.I = 513
+    assert lib.dwarf_linear_wgrad(ctypes.byref(w), None) == L.DWARF_ERR_UNSUPPORTED
+    w.I, w.x_stride = 512, 504
+    assert lib.dwarf_linear_wgrad(ctypes.byref(w), None) == L.DWARF_ERR_UNSUPPORTED   # rows that overlap
+    assert lib.dwarf_linear_wgrad(None, None) == bad

@@ -262,6 +262,58 @@ def test_block_as_one_node_equals_the_composed_block(pkg, device, H, N, lattice,
         assert float((a.double() - b.double()).abs().max()) <= 2.0 ** -7 * scale, n
 
 
+@pytest.mark.parametrize("M,O,I,bias", [(1, 8, 8, True), (65, 136, 264, True), (127, 128, 256, False),
+                                        (129, 2048, 64, True), (700, 72, 520, True), (9000, 512, 512, True)])
+def test_linear_wgrad(pkg, device, M, O, I, bias):
+    """dY^T X and the column sums of dY against float64: one row, rows past a 64-row step by one, outputs and inputs
+    past a 128 x 256 tile by 8, several splits; dY and X as column blocks of wider rows.  Products of bf16 values are
+    exact in float32; M summands in float32 give at most M 2^-24 of the magnitudes' sum, and a random walk of
+    roundings far less: the bar is 2e-6 of that sum."""
+    g = torch.Generator().manual_seed(M + O)
+    dy = torch.randn(M, O + 24, generator=g).to(torch.bfloat16).to(device)[:, 8:8 + O]
+    x = torch.randn(M, I + 8, generator=g).to(torch.bfloat16).to(device)[:, :I]
+    dw, db = pkg.block.linear_wgrad(dy, x, bias)
+    again, _ = pkg.block.linear_wgrad(dy, x, bias)
+    a, b = dy.double().cpu(), x.double().cpu()
+    assert torch.equal(dw, again)
+    assert ((dw.double().cpu() - a.t() @ b).abs() <= 2e-6 * (a.abs().t() @ b.abs())).all()
+    if bias:
+        assert ((db.double().cpu() - a.sum(0)).abs() <= 2e-6 * a.abs().sum(0)).all()
+    else:
+        assert db is None
+
+
+@pytest.mark.parametrize("frozen", ["x", "weights"])
+def test_block_node_with_frozen_parts(pkg, device, frozen):
+    """Gradients that are not needed are not formed and change no other: a block input without gradient, frozen
+    projections; an input in fp32 gets its gradient in fp32."""
+    offsets = list(pkg.lattice.build_offset_groups(2048)[1])
+    blk = StandInBlock(128, 2, offsets, sum(d <= 28 for d in offsets), 2, 64, seed=5).to(device)
+    g = torch.Generator().manual_seed(2)
+    x = torch.randn(2, 70, 128, generator=g).to(device).requires_grad_(True)
+    dy = torch.randn(2, 70, 128, generator=g).to(torch.bfloat16).to(device)
+
+    def step():
+        for p in [x] + list(blk.parameters()):
+            p.grad = None
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            out = pkg.dsqg_block_forward(blk, x)
+        out.backward(dy)
+        return {n: p.grad for n, p in [("x", x)] + list(blk.named_parameters())}
+
+    full = {n: None if t is None else t.clone() for n, t in step().items()}
+    assert full["x"].dtype == torch.float32 and full["qkvg_proj.weight"].dtype == torch.float32
+    gone = ["x"] if frozen == "x" else ["qkvg_proj.weight", "qkvg_proj.bias", "out_proj.weight"]
+    for n in gone:
+        (x if n == "x" else dict(blk.named_parameters())[n]).requires_grad_(False)
+    part = step()
+    for n, t in full.items():
+        if n in gone:
+            assert part[n] is None
+        elif t is not None:
+            assert torch.equal(part[n], t), n
+
+
 def test_block_one_node_compiles(pkg, device):
     """torch.compile traces the block's node with fullgraph and gives the eager bits."""
     offsets = list(pkg.lattice.build_offset_groups(2048)[0])
