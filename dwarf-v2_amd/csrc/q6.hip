@@ -1125,6 +1125,14 @@ constexpr int kMaxDecOffsets = 256;   // offsets the decode step takes
 // waves per CU instead of 24), two 43.2 / 48.2 / 53.6, one 43.4 / 48.1 / 53.0
 constexpr int kDecHeadsPerWg = 4;
 
+constexpr int kDecSplitWaves = 4;     // waves that share a head's list in the split step
+// (sequence, layer, head) items up to which a step is split.  Nine layers of eight
+// heads, 96 offsets, device time against the table's two launches: 1 sequence
+// 4.7 / 11.5 us, 5 5.4 / 11.7, 14 7.1 / 12.0, 28 (2016 items) 11.2 / 13.2, 42
+// (3024) 15.8 / 14.9, 128 41 / 25.5; 28 sequences of 300 tokens 10.3 / 11.9, of
+// 2048 with two KV heads 12.1 / 14.2.
+constexpr int kDecSplitItems = 2048;
+
 struct DecBatch {
   uint32_t k0, k1, k2, v0, v1, v2;
   uint32_t ks, vs;   // fp16 scale pairs of the two groups
@@ -1132,6 +1140,11 @@ struct DecBatch {
   float t;           // the row's T entry: log2(e) (<q, e_j> / 8 + pb_j)
   int j;
   bool ok;
+};
+
+// A batch of the split step: also the lane's 16 dims of the row's E entry, and its pos_bias.
+struct DecSplitBatch : DecBatch {
+  uint4 e[4];
 };
 
 struct DecLayout {
@@ -1259,7 +1272,15 @@ __global__ __launch_bounds__(kBlock) void q6_decode_table(const dwarf_dsqg_q6_de
 // Sum over all 64 lanes, in every lane.
 __device__ __forceinline__ float wave_allsum(float x) { return sum_over_queries16(group_sum<4>(x)); }
 
-template <int SHIFT>
+// SPLIT: the step for few (sequence, layer, head) items (launch_q6_decode has
+// the rule).  A step of few items is its chain of memory round trips: the
+// table launch, then a wave's six batches.  Here a workgroup's four waves share
+// one head's list, wave w taking batches w, w + 4, ..., and each row's
+// <q, e_j> is formed beside its q.k from the E row (bf16, hi and lo for the
+// fp32 table), so there is no table launch and at most two batches in turn;
+// the waves join through LDS.  For many items that costs more than the table
+// (eight v_dot2, eight conversions and four loads a row).
+template <int SHIFT, bool SPLIT>
 __global__ __launch_bounds__(kWave * kMaxDecHeads) void q6_decode_q4(const dwarf_dsqg_q6_decode_args a,
                                                                     const float* __restrict__ T) {
   constexpr float kC = 0.125f * kLog2e;
@@ -1270,14 +1291,14 @@ __global__ __launch_bounds__(kWave * kMaxDecHeads) void q6_decode_q4(const dwarf
   extern __shared__ float smem[];
   int2* s_list_all = reinterpret_cast<int2*>(smem);
 
-  constexpr int HPW = kDecHeadsPerWg;
+  constexpr int HPW = SPLIT ? 1 : kDecHeadsPerWg;   // heads per workgroup
   const int hgroups = (H + HPW - 1) / HPW;
   const int hg = blockIdx.x % hgroups;
   const int sl = blockIdx.x / hgroups;
   const int sq = sl / a.L;
   const int ly = sl - sq * a.L;
   const int wv = uniform(threadIdx.x / kWave);
-  const int h = hg * HPW + wv;   // head = wave index within the group
+  const int h = SPLIT ? hg : hg * HPW + wv;   // head = wave index within the group
   if (h >= H) return;
   const int l = threadIdx.x % kWave;
   const int c = l & 3;        // 16-dim chunk
@@ -1334,7 +1355,13 @@ __global__ __launch_bounds__(kWave * kMaxDecHeads) void q6_decode_q4(const dwarf
       a.J_large > 0 ? (a.J_large - 1) * pg_step + 4 * kPlanes : 0, 0x00020000);
   const bool khi = c >= 2;    // K/V group of this chunk: scale in the high half of the pair
 
-  auto fetch = [&](int k0, DecBatch& b) {
+  using Batch = std::conditional_t<SPLIT, DecSplitBatch, DecBatch>;
+  const int se1 = static_cast<int>(a.se_stride[1]) * 4;   // E row bytes
+  const __amdgpu_buffer_rsrc_t rse = rows_rsrc(a.scale_embed + ly * a.se_stride[0], se1, J, 256);
+  const int pb1 = static_cast<int>(a.pb_stride[1]) * 4, pb2 = static_cast<int>(a.pb_stride[2]) * 4;
+  const __amdgpu_buffer_rsrc_t rpos = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<float*>(a.pos_bias + ly * a.pb_stride[0]), 0, (J - 1) * pb1 + (H - 1) * pb2 + 4, 0x00020000);
+  auto fetch = [&](int k0, Batch& b) {
     const int2 e = list[k0 + rr];
     b.j = e.x;
     const int row = t - e.y;
@@ -1351,11 +1378,19 @@ __global__ __launch_bounds__(kWave * kMaxDecHeads) void q6_decode_q4(const dwarf
     const int i = e.x - J_small;
     b.base = buf_load_f32(rpb, far ? static_cast<uint32_t>(i * ph_step + 4 * c) : kOutOfRange);
     b.gain = buf_load_f32(rpg, far ? static_cast<uint32_t>(i * pg_step + 4 * c) : kOutOfRange);
-    b.t = Th[e.x];
+    if constexpr (SPLIT) {   // the sentinel's E row lies past the table (zeros); its score is not used
+      b.t = buf_load_f32(rpos, e.x < J ? static_cast<uint32_t>(e.x * pb1 + h * pb2) : kOutOfRange);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) b.e[i] = buf_load16(rse, static_cast<uint32_t>(e.x * se1 + 64 * c + 16 * i));
+    } else {
+      b.t = Th[e.x];
+    }
   };
 
-  DecBatch b0, b1;
-  if (cnt > 0) fetch(0, b0);
+  constexpr int kWavesD = SPLIT ? kDecSplitWaves : 1;   // waves that share the list
+  const int first = SPLIT ? kDecRows * wv : 0, step = kDecRows * kWavesD;
+  Batch b0, b1;
+  if (first < cntp) fetch(first, b0);
 
   // this head's query: lane c's 16 dims as bf16 pairs, their sum, and y of
   // plane c = <q, probe_c> / sqrt(|q|^2 + 1e-6 hd) (dsqg:3231-3249)
@@ -1377,10 +1412,24 @@ __global__ __launch_bounds__(kWave * kMaxDecHeads) void q6_decode_q4(const dwarf
   for (int d = 0; d < 16; ++d) acc[d] = 0.f;
   float m = -3.0e38f, lsum = 0.f;
 
-  auto consume = [&](int k0, const DecBatch& b) {
+  auto consume = [&](int k0, const Batch& b) {
     const float kd = q6_dot16_biased(q32, b.k0, b.k1, b.k2) + qbias;
-    const float dot = group_sum<4>(kd * half_lo_or_hi(b.ks, khi));
-    const float s2 = b.ok ? fmaf(dot, kC, b.t) : -INFINITY;
+    float part = kd * half_lo_or_hi(b.ks, khi), add = b.t;
+    if constexpr (SPLIT) {
+      float qe = 0.f;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const float x = __uint_as_float(i & 1 ? b.e[i >> 1].z : b.e[i >> 1].x);
+        const float y = __uint_as_float(i & 1 ? b.e[i >> 1].w : b.e[i >> 1].y);
+        const uint32_t hi = pack_bf16x2(x, y);
+        qe = dot2bf(q32[i], hi, qe);
+        if (!a.se_round_bf16) qe = dot2bf(q32[i], pack_bf16x2(x - bf16_lo(hi), y - bf16_hi(hi)), qe);
+      }
+      part += qe;
+      add *= kLog2e;
+    }
+    const float dot = group_sum<4>(part);
+    const float s2 = b.ok ? fmaf(dot, kC, add) : -INFINITY;
     if (s2 > m + kSlack2) {   // per row group; the groups are put on one scale at the end
       const float f = __builtin_amdgcn_exp2f(m - s2);
 #pragma unroll
@@ -1408,7 +1457,14 @@ __global__ __launch_bounds__(kWave * kMaxDecHeads) void q6_decode_q4(const dwarf
     pin_regs<16>(acc);
   };
 
-  if (cnt > 0) {
+  if constexpr (SPLIT) {   // uniform conditions: the list ends at cntp
+    for (int k0 = first; k0 < cntp; k0 += 2 * step) {
+      if (k0 + step < cntp) fetch(k0 + step, b1);
+      consume(k0, b0);
+      if (k0 + 2 * step < cntp) fetch(k0 + 2 * step, b0);
+      if (k0 + step < cntp) consume(k0 + step, b1);
+    }
+  } else if (cnt > 0) {
     for (int k0 = 0; k0 < cntp; k0 += 2 * kDecRows) {
       fetch(k0 + kDecRows, b1);
       consume(k0, b0);
@@ -1438,9 +1494,29 @@ __global__ __launch_bounds__(kWave * kMaxDecHeads) void q6_decode_q4(const dwarf
       o[i] = x;
     }
   }
+  const int d0 = 16 * c + 8 * (l >> 5) + 4 * ((l >> 4) & 1);
+  if constexpr (SPLIT) {   // the four waves, in order, on the largest reference
+    __shared__ float2 s_ml[kDecSplitWaves];
+    __shared__ __align__(16) float s_o[kDecSplitWaves][kHeadDim];
+    if (l == 0) s_ml[wv] = make_float2(M, lsum);
+    if ((rr & 3) == 0) *reinterpret_cast<float4*>(&s_o[wv][d0]) = make_float4(o[0], o[1], o[2], o[3]);
+    __syncthreads();
+    if (wv > 0) return;
+    float top = s_ml[0].x;
+#pragma unroll
+    for (int u = 1; u < kDecSplitWaves; ++u) top = fmaxf(top, s_ml[u].x);
+    lsum = 0.f;
+    o[0] = o[1] = o[2] = o[3] = 0.f;
+#pragma unroll
+    for (int u = 0; u < kDecSplitWaves; ++u) {
+      const float f = __builtin_amdgcn_exp2f(s_ml[u].x - top);
+      const float4 x = *reinterpret_cast<const float4*>(&s_o[u][d0]);
+      lsum = fmaf(s_ml[u].y, f, lsum);
+      o[0] = fmaf(x.x, f, o[0]); o[1] = fmaf(x.y, f, o[1]); o[2] = fmaf(x.z, f, o[2]); o[3] = fmaf(x.w, f, o[3]);
+    }
+  }
   if ((rr & 3) == 0) {
     const float inv = lsum > 0.f ? 1.f / lsum : 0.f;
-    const int d0 = 16 * c + 8 * (l >> 5) + 4 * ((l >> 4) & 1);
     uint2 x;
     x.x = pack_bf16x2(o[0] * inv, o[1] * inv);
     x.y = pack_bf16x2(o[2] * inv, o[3] * inv);
@@ -1540,15 +1616,23 @@ size_t q6_decode_workspace(const dwarf_dsqg_q6_decode_args& a) {
 
 hipError_t launch_q6_decode(const dwarf_dsqg_q6_decode_args& a, float* T, hipStream_t stream) {
   const DecLayout lay = dec_layout(a.J, a.H);
-  const int table_blocks = a.L * ((a.S * a.H + kTabRows - 1) / kTabRows);
-  hipLaunchKernelGGL(q6_decode_table, dim3(table_blocks), dim3(kBlock), dec_table_lds(lay.JE, a.H, !a.se_round_bf16),
-                     stream, a, T, lay.JE);
-  constexpr int HPW = kDecHeadsPerWg;
-  const int wpb = a.H < HPW ? a.H : HPW;
-  const int blocks = a.S * a.L * ((a.H + HPW - 1) / HPW);
-  const size_t lds = static_cast<size_t>(wpb) * lay.list_len * 8;
-#define DWARF_Q6D_CASE(S) \
-  case S: hipLaunchKernelGGL(q6_decode_q4<S>, dim3(blocks), dim3(kWave * wpb), lds, stream, a, T); break;
+  const bool split = static_cast<int64_t>(a.S) * a.L * a.H <= kDecSplitItems;
+  if (!split) {
+    const int table_blocks = a.L * ((a.S * a.H + kTabRows - 1) / kTabRows);
+    hipLaunchKernelGGL(q6_decode_table, dim3(table_blocks), dim3(kBlock), dec_table_lds(lay.JE, a.H, !a.se_round_bf16),
+                       stream, a, T, lay.JE);
+  }
+  const int heads = split ? 1 : (a.H < kDecHeadsPerWg ? a.H : kDecHeadsPerWg);   // per workgroup
+  const int waves = split ? kDecSplitWaves : heads;
+  const int blocks = a.S * a.L * ((a.H + (split ? 1 : kDecHeadsPerWg) - 1) / (split ? 1 : kDecHeadsPerWg));
+  const size_t lds = static_cast<size_t>(waves) * lay.list_len * 8;
+#define DWARF_Q6D_CASE(S)                                                                                           \
+  case S:                                                                                                           \
+    if (split)                                                                                                      \
+      hipLaunchKernelGGL((q6_decode_q4<S, true>), dim3(blocks), dim3(kWave * waves), lds, stream, a, T);            \
+    else                                                                                                            \
+      hipLaunchKernelGGL((q6_decode_q4<S, false>), dim3(blocks), dim3(kWave * waves), lds, stream, a, T);           \
+    break;
   switch (a.plane_shift) {
     DWARF_Q6D_CASE(0) DWARF_Q6D_CASE(1) DWARF_Q6D_CASE(2) DWARF_Q6D_CASE(3) DWARF_Q6D_CASE(4)
     DWARF_Q6D_CASE(5) DWARF_Q6D_CASE(6) DWARF_Q6D_CASE(7) DWARF_Q6D_CASE(8) DWARF_Q6D_CASE(9)

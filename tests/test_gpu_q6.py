@@ -282,6 +282,36 @@ def test_decode_maximum_sizes(pkg, device):
         assert max_abs(out[s, 0], ref[s, :, int(pos[s])]) < 2e-2, s
 
 
+@pytest.mark.parametrize("far,round_se", [(79, True), (79, False), (239, True)])
+@pytest.mark.parametrize("split", [True, False])
+def test_decode_split_rule(pkg, device, split, far, round_se):
+    """Up to 2048 (sequence, layer, head) items four waves share a head's list and form <q, e_j> as they go, above that
+    a wave takes a head and reads the table: the same six sequences (no valid offset, one, near ones only, the last
+    batch of one row, all valid) repeated to the last count of the one kernel and the first of the other, each copy
+    against the oracle on the dequantised cache.  SE is scaled up where it stays fp32, so that its rounding would show."""
+    offsets = list(range(1, 18)) + list(range(48, 48 + 239)) if far == 239 else list(pkg.ALL_OFFSETS)
+    H, N = 8, 320
+    x = make_inputs(6, H, 4, N, offsets, 17, seed=140 + far, dtype=torch.bfloat16, plane_shift=1, gain_std=6.0)
+    if not round_se:
+        x["scale_embed"] = 40.0 * x["scale_embed"]
+    pos = torch.tensor([0, 1, 30, 64, 257, 319], dtype=torch.int32)
+    qp, kp = (torch.nn.functional.normalize(t, dim=-1) for t in orthogonal_probes(64, 1))
+    cache = pkg.q6.pack_kv(x["k"].to(device), x["v"].to(device), kp.to(device))
+    S = 256 if split else 257
+    seq = torch.arange(S) % 6
+    qdec = x["q"][seq, :, pos[seq].long()].unsqueeze(1)
+    tab = {n: x[n].unsqueeze(0).to(device) for n in ("pos_bias", "scale_embed", "phase_base", "phase_gain")}
+    off = torch.tensor(offsets, dtype=torch.int32, device=device)
+    out = pkg.q6.q6_decode(qdec.to(device), pos[seq].to(device), cache[seq.to(device)].unsqueeze(0), tab["pos_bias"],
+                           tab["scale_embed"], tab["phase_base"], tab["phase_gain"], qp.unsqueeze(0).to(device), off,
+                           17, far, 1, round_se=round_se).cpu()
+    ref = _oracle_on_cache(x, cache.cpu().numpy(), offsets, 17, 1, qp, kp, 0, round_se=round_se)
+    assert not out[seq == 0].any()
+    for s in range(6):
+        assert torch.equal(out[seq == s], out[s:s + 1].expand(int((seq == s).sum()), -1, -1, -1)), s
+        assert max_abs(out[s, 0], ref[s, :, int(pos[s])]) < 2e-2, s
+
+
 @pytest.mark.parametrize("H,Hkv", [(3, 3), (6, 3)])
 def test_decode_head_groups(pkg, device, H, Hkv):
     """A decode workgroup takes four heads: H = 3 is one workgroup of three waves; H = 6 (GQA, two query
