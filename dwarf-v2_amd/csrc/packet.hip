@@ -963,7 +963,8 @@ template <typename T, typename G, int VEC>
 __global__ __launch_bounds__(kPkRowMaxThreads) void packet_bwd_rows(
     const T* __restrict__ pooled, int64_t spb, int64_t spn, const float* __restrict__ ms,
     const G* __restrict__ gate, int64_t sgb, int64_t sgn, const G* __restrict__ dpacket, int64_t sdb, int64_t sdn,
-    T* __restrict__ dpooled, int64_t sab, int64_t san, G* __restrict__ dgate, int64_t seb, int64_t sen, EmaGeom g) {
+    T* __restrict__ dpooled, int64_t sab, int64_t san, G* __restrict__ dgate, int64_t seb, int64_t sen,
+    uint4* __restrict__ words, int64_t n16, EmaGeom g) {
   __shared__ float s_red[kPkBwdTokens][kPkRowMaxThreads / kWave];
   __shared__ float s_sum[kPkBwdTokens];
   const int groups = (g.N + kPkBwdTokens - 1) / kPkBwdTokens;
@@ -973,6 +974,9 @@ __global__ __launch_bounds__(kPkRowMaxThreads) void packet_bwd_rows(
   const int dv = threadIdx.x;
   const bool live = dv < g.DV;
   const int d0 = dv * VEC;
+  for (int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < n16;
+       i += static_cast<int64_t>(gridDim.x) * blockDim.x)
+    words[i] = make_uint4(0u, 0u, 0u, 0u);   // the look-back words of packet_bwd_lb, which follows
   float u[kPkBwdTokens][VEC], dp[kPkBwdTokens][VEC], sg[kPkBwdTokens][VEC];
   float part[kPkBwdTokens];
 #pragma unroll
@@ -1157,11 +1161,11 @@ void pkt_fwd_typed(const dwarf_packet_fwd_args& p, hipStream_t stream) {
 }
 
 // The backward in one pass where every [N][D] slab of x, dpooled and dx spans
-// less than 2 GiB: the words' zeroing launch, packet_bwd_lb, then the
-// parameter sums over its workgroups' slots.  False: the three-stage
-// backward runs instead.
+// less than 2 GiB: the words' zeroing launch (unless the caller has cleared
+// them), packet_bwd_lb, then the parameter sums over its workgroups' slots.
+// False: the three-stage backward runs instead.
 template <typename T, int VEC, int K, int KT, int SEG>
-bool pk_bwd_lookback(const dwarf_packet_pool_bwd_args& a, hipStream_t stream) {
+bool pk_bwd_lookback(const dwarf_packet_pool_bwd_args& a, bool cleared, hipStream_t stream) {
   const dwarf_packet_pool_fwd_args& f = a.fwd;
   if (!lb_fits(f.N, f.x_stride[1], sizeof(T)) || !lb_fits(f.N, a.dpooled_stride[1], sizeof(T)) ||
       !lb_fits(f.N, a.dx_stride[1], sizeof(T)))
@@ -1170,7 +1174,7 @@ bool pk_bwd_lookback(const dwarf_packet_pool_bwd_args& a, hipStream_t stream) {
   const LbGeom g = pk_lb_geom(f.B, f.N, f.D, K, f.floor_, f.ceiling, a.workspace, p);
   float* part = reinterpret_cast<float*>(static_cast<char*>(a.workspace) + kLbHead + pk_round256(p.words_bytes));
   const int slots = p.NWG * p.S;
-  lb_zero(g, p, stream);
+  if (!cleared) lb_zero(g, p, stream);
   hipLaunchKernelGGL((packet_bwd_lb<T, VEC, K, KT, SEG>), dim3(slots), dim3(kWave * kLbWaves), 0, stream,
                      static_cast<const T*>(f.x), f.x_stride[0], f.x_stride[1], static_cast<const T*>(a.dpooled),
                      a.dpooled_stride[0], a.dpooled_stride[1], static_cast<T*>(a.dx), a.dx_stride[0], a.dx_stride[1],
@@ -1184,12 +1188,14 @@ bool pk_bwd_lookback(const dwarf_packet_pool_bwd_args& a, hipStream_t stream) {
 }
 
 
+// Channels per lane of packet_bwd_lb: four up to three scales (four scales there overflow the registers into
+// scratch memory), else one.
+constexpr int pk_bwd_lb_vec(int vec, int K) { return vec == 4 && K <= 3 ? 4 : 1; }
+
 template <typename T, int VEC, int VA, int K>
-void pk_bwd_typed(const dwarf_packet_pool_bwd_args& a, hipStream_t stream) {
-  // four channels per lane up to three scales (four scales there overflow the registers into scratch
-  // memory), else one
-  constexpr int LBV = VEC == 4 && K <= 3 ? 4 : 1;
-  if (pk_bwd_lookback<T, LBV, K, LBV == 4 ? pk_lb_keep<T>() : kChunkT, kPkLbSeg>(a, stream)) return;
+void pk_bwd_typed(const dwarf_packet_pool_bwd_args& a, bool cleared, hipStream_t stream) {
+  constexpr int LBV = pk_bwd_lb_vec(VEC, K);
+  if (pk_bwd_lookback<T, LBV, K, LBV == 4 ? pk_lb_keep<T>() : kChunkT, kPkLbSeg>(a, cleared, stream)) return;
   const dwarf_packet_pool_fwd_args& f = a.fwd;
   const size_t nf = pk_state_floats(f.B, f.N, f.D, K);
   float* starts = static_cast<float*>(a.workspace);
@@ -1226,12 +1232,12 @@ void pk_fwd_k(const dwarf_packet_pool_fwd_args& a, hipStream_t s) {
 }
 
 template <typename T, int VEC, int VA>
-void pk_bwd_k(const dwarf_packet_pool_bwd_args& a, hipStream_t s) {
+void pk_bwd_k(const dwarf_packet_pool_bwd_args& a, bool cleared, hipStream_t s) {
   switch (a.fwd.K) {
-    case 1: pk_bwd_typed<T, VEC, VA, 1>(a, s); break;
-    case 2: pk_bwd_typed<T, VEC, VA, 2>(a, s); break;
-    case 3: pk_bwd_typed<T, VEC, VA, 3>(a, s); break;
-    default: pk_bwd_typed<T, VEC, VA, 4>(a, s); break;
+    case 1: pk_bwd_typed<T, VEC, VA, 1>(a, cleared, s); break;
+    case 2: pk_bwd_typed<T, VEC, VA, 2>(a, cleared, s); break;
+    case 3: pk_bwd_typed<T, VEC, VA, 3>(a, cleared, s); break;
+    default: pk_bwd_typed<T, VEC, VA, 4>(a, cleared, s); break;
   }
 }
 
@@ -1247,6 +1253,9 @@ void pkt_fwd_k(const dwarf_packet_fwd_args& a, hipStream_t s) {
 
 // The packet's backward: dpooled (into the workspace after the pool's part)
 // and dgate from the rows kernel, then the pool's backward on that dpooled.
+// The rows kernel also clears the pool backward's look-back words, whose
+// launch of their own took 4.7 us at [15, 2048, 512] bf16 (forward and backward 150.5 us with it, 148.0 without) (where the three-stage
+// backward follows, it only writes over them).
 template <typename T, typename G, int VEC, int VA>
 void pkt_bwd_k(const dwarf_packet_bwd_args& p, hipStream_t s) {
   const dwarf_packet_pool_fwd_args& f = p.fwd.pool;
@@ -1256,11 +1265,14 @@ void pkt_bwd_k(const dwarf_packet_bwd_args& p, hipStream_t s) {
   const int64_t dsn = f.D, dsb = static_cast<int64_t>(f.N) * f.D;
   const int nt = pk_row_threads(g.DV);
   const int groups = (f.N + kPkBwdTokens - 1) / kPkBwdTokens;
+  const LbPlan lb = lb_plan(f.B, f.N, f.D, pk_bwd_lb_vec(VEC, f.K), kPkLbSeg, f.K);
   hipLaunchKernelGGL((packet_bwd_rows<T, G, VEC>), dim3(f.B * groups), dim3(nt), 0, s,
                      static_cast<const T*>(f.pooled), f.pooled_stride[0], f.pooled_stride[1], p.fwd.ms,
                      static_cast<const G*>(p.fwd.gate), p.fwd.gate_stride[0], p.fwd.gate_stride[1],
                      static_cast<const G*>(p.dpacket), p.dpacket_stride[0], p.dpacket_stride[1], dpooled, dsb, dsn,
-                     static_cast<G*>(p.dgate), p.dgate_stride[0], p.dgate_stride[1], g);
+                     static_cast<G*>(p.dgate), p.dgate_stride[0], p.dgate_stride[1],
+                     reinterpret_cast<uint4*>(static_cast<char*>(p.workspace) + kLbHead),
+                     static_cast<int64_t>(lb.words_bytes / 16), g);
   dwarf_packet_pool_bwd_args pb{};
   pb.fwd = f;
   pb.dpooled = dpooled;
@@ -1271,7 +1283,7 @@ void pkt_bwd_k(const dwarf_packet_bwd_args& p, hipStream_t s) {
   pb.dweight = p.dweight;
   pb.workspace = p.workspace;
   pb.workspace_bytes = pool_ws;
-  pk_bwd_k<T, VEC, VA>(pb, s);
+  pk_bwd_k<T, VEC, VA>(pb, true, s);
 }
 
 }  // namespace
@@ -1311,11 +1323,11 @@ hipError_t launch_packet_fwd(const dwarf_packet_pool_fwd_args& a, hipStream_t st
 hipError_t launch_packet_bwd(const dwarf_packet_pool_bwd_args& a, hipStream_t stream) {
   const bool vec4 = (a.fwd.D % 4) == 0;
   if (a.fwd.dtype == DWARF_BF16) {
-    if (vec4) pk_bwd_k<bf16, 4, 2>(a, stream);
-    else pk_bwd_k<bf16, 1, 1>(a, stream);
+    if (vec4) pk_bwd_k<bf16, 4, 2>(a, false, stream);
+    else pk_bwd_k<bf16, 1, 1>(a, false, stream);
   } else {
-    if (vec4) pk_bwd_k<float, 4, 1>(a, stream);
-    else pk_bwd_k<float, 1, 1>(a, stream);
+    if (vec4) pk_bwd_k<float, 4, 1>(a, false, stream);
+    else pk_bwd_k<float, 1, 1>(a, false, stream);
   }
   return hipGetLastError();
 }

@@ -280,6 +280,28 @@ def test_packet_matches_oracle(pkg, device, dtype, gdtype, B, N, D, K):
         assert rel_err(dw, rdw) < 1e-2
 
 
+@pytest.mark.parametrize("K,D", [(3, 64), (4, 64), (3, 30)])
+def test_packet_backward_clears_the_lookback_words(pkg, device, K, D):
+    """The backward's rows kernel clears the look-back words of the pool pass that follows it: with memory that held
+    valid-looking words (tag 1, value 100) where the workspace comes from, the gradients are the oracle's, and the same
+    bits as from zeroed memory.  Four channels per lane, one (four scales), one (D not a multiple of four); 1100 tokens
+    are three workgroups per slice."""
+    B, N = 2, 1100
+    x, a, w, gate, dpk = packet_inputs(B, N, D, K, torch.float32, torch.float32, seed=31 + K + D)
+    xd, ad, wd, gd, pd = (t.to(device) for t in (x, a, w, gate, dpk))
+    _, pooled, state, ms = pkg.packet.packet_forward(xd, ad, wd, gd, 1e-5, 0.5)
+    got = []
+    for word in (0, (1 << 32) | 0x42C80000):
+        junk = [torch.full((n,), word, dtype=torch.int64, device=device) for n in (1 << 18, 1 << 19, 1 << 20) * 4]
+        torch.cuda.synchronize()
+        del junk
+        got.append([t.cpu() for t in pkg.packet.packet_backward(xd, ad, wd, gd, pooled, state, ms, pd, 1e-5, 0.5)])
+    assert all(torch.equal(u, v) for u, v in zip(*got))
+    _, rdx, rda, rdw, rdg = packet_oracle(x, a, w, gate, pooled.cpu(), dpk)
+    for g, r in zip(got[0], (rdx, rda, rdw, rdg)):
+        assert rel_err(g, r) < 1e-5
+
+
 def test_packet_deterministic_compile_and_graph(pkg, device):
     """interference_packet twice bit-equal, under torch.compile (fullgraph) bit-equal to eager, and its raw
     forward + backward launches replayed from a HIP graph equal to eager on every replay."""
