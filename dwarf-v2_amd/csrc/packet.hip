@@ -1253,9 +1253,10 @@ void pkt_fwd_k(const dwarf_packet_fwd_args& a, hipStream_t s) {
 
 // The packet's backward: dpooled (into the workspace after the pool's part)
 // and dgate from the rows kernel, then the pool's backward on that dpooled.
-// The rows kernel also clears the pool backward's look-back words, whose
-// launch of their own took 4.7 us at [15, 2048, 512] bf16 (forward and backward 150.5 us with it, 148.0 without) (where the three-stage
-// backward follows, it only writes over them).
+// The rows kernel also clears the pool backward's look-back words: a launch of
+// their own took 4.7 us (forward and backward at [15, 2048, 512] bf16 150.5 us
+// with it, 148.0 without).  Where the three-stage backward follows, it only
+// writes over them.
 template <typename T, typename G, int VEC, int VA>
 void pkt_bwd_k(const dwarf_packet_bwd_args& p, hipStream_t s) {
   const dwarf_packet_pool_fwd_args& f = p.fwd.pool;

@@ -2,8 +2,8 @@
  * Entry points for the DSQG block around the attention op (libdwarf_dsqg.so,
  * gfx950): the normalised phase probes, the backward's two streams in one
  * call, the per-head gain and content gate after the attention, forward and
- * backward, and the projections' weight gradients.  Conventions (status codes, strides in elements, dwarf_stream_t)
- * are those of dwarf_dsqg.h.
+ * backward, and the projections' weight gradients.  Conventions (status
+ * codes, strides in elements, dwarf_stream_t) are those of dwarf_dsqg.h.
  */
 #ifndef DWARF_BLOCK_H
 #define DWARF_BLOCK_H
