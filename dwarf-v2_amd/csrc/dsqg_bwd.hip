@@ -565,8 +565,19 @@ hipError_t launch_dkdv_bf16_k4(const dwarf_dsqg_bwd_args& a, const BwdWorkspace&
 }
 
 // ---------------------------------------------------------------------------
-// Fixed-order reduction of the parameter-gradient partials.
+// Fixed-order reduction of the parameter-gradient partials: groups of kRedRows
+// rows summed in row order, then the groups in order.  One launch
+// (dsqg_bwd_reduce) up to kRedOneLaunch groups, a wave to a group of 64
+// columns joined through LDS; two launches above, which give the same bits.
+// What a small sum costs is its launches and round trips, so one launch takes
+// 3-4 us off the backward at one sequence of 2,048 tokens (75.0 -> 71.2 us,
+// serial 105.9 -> 103.5, fp32 107.5 -> 103.7) and at 15 (470 -> 457, 471 ->
+// 469; 8 groups); at 60 (30 groups) it is even (1,660), and at 120 (60) the
+// more workgroups of the first of two launches are worth it (3,249 / 3,257).
+// Four and 16 waves measured as eight do.
 // ---------------------------------------------------------------------------
+constexpr int kRedOneLaunch = 32;   // groups up to which one launch reduces
+constexpr int kRedWaves = 8;
 constexpr int kRedRows = 64;  // rows summed per stage-1 group (16 rows: the step 3-4 us longer at B15 H8 T2048)
 
 struct RedArray {
@@ -601,16 +612,8 @@ __global__ __launch_bounds__(kBlock) void dsqg_bwd_reduce1(RedPlan p) {
   A.tmp[(static_cast<int64_t>(seg) * A.groups + grp) * A.cols + col] = sum;
 }
 
-__global__ __launch_bounds__(kBlock) void dsqg_bwd_reduce2(RedPlan p, const dwarf_dsqg_bwd_args a) {
-  int idx = blockIdx.x * kBlock + threadIdx.x, ai = 0;
-  while (ai < 2 && idx >= p.outputs[ai]) idx -= p.outputs[ai++];
-  if (idx >= p.outputs[ai]) return;
-  const RedArray& A = p.arr[ai];
-  const int seg = idx / A.cols, col = idx - seg * A.cols;
-  const float* src = A.tmp + static_cast<int64_t>(seg) * A.groups * A.cols + col;
-  float sum = 0.f;
-#pragma unroll 8
-  for (int gi = 0; gi < A.groups; ++gi, src += A.cols) sum += *src;
+// Output `col` of segment seg of array ai.
+__device__ __forceinline__ void red_store(const dwarf_dsqg_bwd_args& a, int ai, int seg, int col, float sum) {
   const dwarf_dsqg_fwd_args& f = a.fwd;
   if (ai == 0) {
     a.dscale_embed[col] = sum;                          // [J][64]
@@ -621,6 +624,44 @@ __global__ __launch_bounds__(kBlock) void dsqg_bwd_reduce2(RedPlan p, const dwar
     float* dst = (rk & 1) ? a.dphase_gain : a.dphase_base;
     dst[(i * f.H + seg) * kPlanes + (rk >> 1)] = sum;   // [J_L][H][4]
   }
+}
+
+__global__ __launch_bounds__(kWave * kRedWaves) void dsqg_bwd_reduce(RedPlan p, const dwarf_dsqg_bwd_args a) {
+  __shared__ float s_part[kRedOneLaunch][kWave];
+  int blk = blockIdx.x, ai = 0;
+  auto blocks = [&](int i) { return p.arr[i].nseg * ((p.arr[i].cols + kWave - 1) / kWave); };
+  while (ai < 2 && blk >= blocks(ai)) blk -= blocks(ai++);
+  const RedArray& A = p.arr[ai];
+  const int cblocks = (A.cols + kWave - 1) / kWave;
+  const int seg = blk / cblocks, lane = threadIdx.x % kWave;
+  const int col = (blk - seg * cblocks) * kWave + lane;
+  const bool live = col < A.cols;
+  for (int grp = threadIdx.x / kWave; grp < A.groups; grp += kRedWaves) {
+    const int r0 = grp * kRedRows, r1 = min(A.rows, r0 + kRedRows);
+    const float* src = A.in + (static_cast<int64_t>(seg) * A.rows + r0) * A.cols + (live ? col : A.cols - 1);
+    float sum = 0.f;
+#pragma unroll 16
+    for (int r = r0; r < r1; ++r, src += A.cols) sum += *src;
+    s_part[grp][lane] = sum;
+  }
+  __syncthreads();
+  if (threadIdx.x >= kWave || !live) return;
+  float sum = 0.f;
+  for (int grp = 0; grp < A.groups; ++grp) sum += s_part[grp][lane];
+  red_store(a, ai, seg, col, sum);
+}
+
+__global__ __launch_bounds__(kBlock) void dsqg_bwd_reduce2(RedPlan p, const dwarf_dsqg_bwd_args a) {
+  int idx = blockIdx.x * kBlock + threadIdx.x, ai = 0;
+  while (ai < 2 && idx >= p.outputs[ai]) idx -= p.outputs[ai++];
+  if (idx >= p.outputs[ai]) return;
+  const RedArray& A = p.arr[ai];
+  const int seg = idx / A.cols, col = idx - seg * A.cols;
+  const float* src = A.tmp + static_cast<int64_t>(seg) * A.groups * A.cols + col;
+  float sum = 0.f;
+#pragma unroll 8
+  for (int gi = 0; gi < A.groups; ++gi, src += A.cols) sum += *src;
+  red_store(a, ai, seg, col, sum);
 }
 
 RedPlan make_red_plan(const dwarf_dsqg_bwd_args& a, const BwdWorkspace& ws) {
@@ -728,10 +769,19 @@ hipError_t launch_dsqg_bwd(const dwarf_dsqg_bwd_args& a, const BwdWorkspace& ws,
     hipError_t e = launch_dsqg_bwd_dse(a, ws, stream);
     if (e != hipSuccess) return e;
     const RedPlan p = make_red_plan(a, ws);
-    const int b1 = p.blocks1[0] + p.blocks1[1] + p.blocks1[2];
-    const int o2 = p.outputs[0] + p.outputs[1] + p.outputs[2];
-    if (b1 > 0) hipLaunchKernelGGL(dsqg_bwd_reduce1, dim3(b1), dim3(kBlock), 0, stream, p);
-    if (o2 > 0) hipLaunchKernelGGL(dsqg_bwd_reduce2, dim3((o2 + kBlock - 1) / kBlock), dim3(kBlock), 0, stream, p, a);
+    int o1 = 0, groups = 0;   // 64-column blocks; a lattice without far offsets leaves dPhase empty
+    for (const RedArray& A : p.arr) {
+      o1 += A.nseg * ((A.cols + kWave - 1) / kWave);
+      if (A.cols > 0 && A.groups > groups) groups = A.groups;
+    }
+    if (groups <= kRedOneLaunch) {
+      if (o1 > 0) hipLaunchKernelGGL(dsqg_bwd_reduce, dim3(o1), dim3(kWave * kRedWaves), 0, stream, p, a);
+    } else {
+      const int b1 = p.blocks1[0] + p.blocks1[1] + p.blocks1[2];
+      const int o2 = p.outputs[0] + p.outputs[1] + p.outputs[2];
+      hipLaunchKernelGGL(dsqg_bwd_reduce1, dim3(b1), dim3(kBlock), 0, stream, p);
+      hipLaunchKernelGGL(dsqg_bwd_reduce2, dim3((o2 + kBlock - 1) / kBlock), dim3(kBlock), 0, stream, p, a);
+    }
     e = hipGetLastError();
     if (e != hipSuccess) return e;
   }

@@ -531,3 +531,28 @@ def test_fp32_masked_offsets_and_foreign_nan(pkg, device):
     assert torch.equal(o2[:, :, ~hit], out[:, :, ~hit])
     assert torch.isnan(o2[:, :, hit]).any(-1).all()
     assert torch.equal(g2["q"][:, :, ~hit], grads["q"][:, :, ~hit])
+
+
+@pytest.mark.parametrize("offsets,js", [([1, 2, 5, 18, 20, 33], 3), ([1, 2, 3], 3)])
+def test_parameter_reduction_rule(pkg, device, offsets, js):
+    """The parameter sums take one launch up to 32 groups of 64 partial rows and two above.  2048 sequences of one tile
+    are the last 32 groups; one more sequence, whose output gradient is zero, adds rows of zeros and the other kernels:
+    dpos_bias and the phase gradients keep their bits, dscale_embed (accumulated per persistent workgroup, so in another
+    order) to fp32 rounding.  At 600 sequences every gradient is the oracle's."""
+    N = 40
+    x = make_inputs(2049, 1, 1, N, offsets, js, seed=5, dtype=torch.bfloat16, plane_shift=1, gain_std=4.0)
+    dout = torch.randn(2049, 1, N, 64, generator=torch.Generator().manual_seed(6)).bfloat16()
+    dout[2048] = 0
+    tables = ("pos_bias", "scale_embed", "phase_base", "phase_gain")
+    grads = {}
+    for B in (2048, 2049, 600):
+        part = {n: t if n in tables else t[:B] for n, t in x.items()}
+        grads[B] = gpu_fwd_bwd(pkg, part, offsets, js, 1, 1, dout[:B], device)[1]
+    for n in ("pos_bias", "phase_base", "phase_gain"):
+        assert torch.equal(grads[2048][n], grads[2049][n]), n
+    assert rel_err(grads[2049]["scale_embed"], grads[2048]["scale_embed"].double().cpu()) < 1e-5
+    part = {n: t if n in tables else t[:600] for n, t in x.items()}
+    _, _, rg = oracle_fwd_bwd(part, offsets, js, 1, 1, dout[:600], round_se=True)
+    for n in tables:
+        if rg[n] is not None:   # None: no far offset takes part
+            assert rel_err(grads[600][n], rg[n]) < BF16_ABS, n
