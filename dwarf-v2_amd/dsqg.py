@@ -39,7 +39,7 @@ DEFAULT_SCHEDULE = _lib.DWARF_SCHED_BAND
 # B15 T2048, 23 far: 6 near 269 / 239, 9 273 / 255, 10 271 / 263, 12 271 / 273, 17 278 / 305; 79 far: 9 454 / 438,
 # 10 450 / 450, 12 454 / 461; B4 T8192, 23 far: 9 354 / 336, 10 351 / 352, 12 355 / 361.  Forward, B15 T2048, 23 far:
 # 3 near 71 / 62, 6 68 / 67, 8 70 / 73, 10 69 / 78; B4 T8192, 79 far: 6 208 / 209, 8 210 / 210, 10 207 / 214.
-BAND_MIN_FORWARD, BAND_MIN_BACKWARD = 7, 11
+BAND_MIN_FORWARD, BAND_MIN_BACKWARD = 6, 11
 
 
 def schedule_for(grouped_mode_id: int, online_softmax: bool, j_small: int | None = None, backward: bool = False) -> int:
