@@ -521,6 +521,7 @@ __global__ __launch_bounds__(kBlock) void dsqg_f32_dse(const dwarf_dsqg_bwd_args
   const int w = threadIdx.x / kWave, l = threadIdx.x % kWave, lr = l & 15, lc = l >> 4;
   const int slot = (h * f.B + b) * n_tg + tg;
   const float* qbase = reinterpret_cast<const float*>(f.q) + b * f.q_stride[0] + h * f.q_stride[1];
+  const float* lbase = f.lse + b * f.lse_stride[0] + h * f.lse_stride[1];
   f32x4 acc[MB][4];
   float pb[MB];
   int off[MB];
@@ -540,12 +541,23 @@ __global__ __launch_bounds__(kBlock) void dsqg_f32_dse(const dwarf_dsqg_bwd_args
       const int j = 16 * (w + kWavesF * m) + lr;
       load16(ds_ws + (static_cast<int64_t>(bh) * J + (j < J ? j : J - 1)) * NP + n0 + 16 * lc, x[m]);
     }
+    // q as zeros for a row without mass: its dS are zeros, which do not keep a NaN or inf out of the products
+    constexpr int kQRows = 64 * 16 / kBlock;   // row pieces per thread
+    float4 qv[kQRows];
+    bool mass[kQRows];
+#pragma unroll
+    for (int u = 0; u < kQRows; ++u) {
+      const int n = n0 + (threadIdx.x >> 4) + u * (kBlock / 16);
+      const int64_t nc = min(n, N - 1);
+      qv[u] = *reinterpret_cast<const float4*>(qbase + nc * f.q_stride[2] + 4 * (threadIdx.x & 15));
+      mass[u] = n < N && n >= f.query_start && lbase[nc * f.lse_stride[2]] > -INFINITY;
+    }
     __syncthreads();   // the previous tile's q has been read
-    for (int i = threadIdx.x; i < 64 * 16; i += kBlock) {
-      const int r = i >> 4, c = 4 * (i & 15);
-      const float4 v = *reinterpret_cast<const float4*>(qbase + static_cast<int64_t>(min(n0 + r, N - 1)) * f.q_stride[2] + c);
-      float* d = s_q + r * kRow + c;
-      d[0] = v.x; d[1] = v.y; d[2] = v.z; d[3] = v.w;
+#pragma unroll
+    for (int u = 0; u < kQRows; ++u) {
+      float* d = s_q + ((threadIdx.x >> 4) + u * (kBlock / 16)) * kRow + 4 * (threadIdx.x & 15);
+      d[0] = mass[u] ? qv[u].x : 0.f; d[1] = mass[u] ? qv[u].y : 0.f;
+      d[2] = mass[u] ? qv[u].z : 0.f; d[3] = mass[u] ? qv[u].w : 0.f;
     }
     __syncthreads();
 #pragma unroll
@@ -657,7 +669,9 @@ __global__ __launch_bounds__(kBlock) void dsqg_f32_dkdv(const dwarf_dsqg_bwd_arg
         for (int r = 0; r < kPlanes; ++r) t[r] = va[r] * wv[r][1] - vv[r] * wv[r][0];
         turn = Pair<SHIFT>::plane(t, g);
       }
-      if (s.ok) {
+      // a query without mass has P = dS = 0, and nothing of its rows may pass (0 times a NaN or inf is NaN); where a
+      // query with mass has both, its terms are zeros
+      if (s.ok && ((__float_as_uint(s.p) | __float_as_uint(s.ds)) << 1) != 0u) {
         const float c = 0.125f * s.ds;
 #pragma unroll
         for (int i = 0; i < kDims; ++i) {

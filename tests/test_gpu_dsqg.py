@@ -533,6 +533,26 @@ def test_fp32_masked_offsets_and_foreign_nan(pkg, device):
     assert torch.equal(g2["q"][:, :, ~hit], grads["q"][:, :, ~hit])
 
 
+@pytest.mark.parametrize("H,Hkv,N", [(2, 2, 200), (4, 2, 131)])
+def test_fp32_rows_without_mass_reach_no_gradient(pkg, device, H, Hkv, N):
+    """NaN and inf in the q, dO and y rows of queries that take no part (before query_start, or with every source
+    masked by a pos_bias of -inf) change no gradient's bits: they are no one's source and no summand."""
+    offsets, js, qs = [1, 2, 5, 48, 64, 130], 3, 3
+    x = make_inputs(2, H, Hkv, N, offsets, js, seed=11, dtype=torch.float32, plane_shift=3)
+    dout = torch.randn(2, H, N, 64, generator=torch.Generator().manual_seed(12))
+    x["pos_bias"][[0, 1, 3]] = float("-inf")   # rows 3 and 4 have sources at 1 and 2 alone
+    out, grads = gpu_fwd_bwd(pkg, x, offsets, js, 3, qs, dout, device)
+    assert not out[:, :, :5].any() and all(torch.isfinite(g).all() for g in grads.values())
+    bad, d2 = {n: t.clone() for n, t in x.items()}, dout.clone()
+    for t in (bad["q"], bad["y_pre"], d2):
+        t[:, :, [0, 2, 3]] = float("nan")
+        t[:, :, [1, 4]] = float("inf")
+    o2, g2 = gpu_fwd_bwd(pkg, bad, offsets, js, 3, qs, d2, device)
+    assert torch.equal(o2[:, :, 5:], out[:, :, 5:])
+    for n in NAMES:
+        assert torch.equal(g2[n], grads[n]), n
+
+
 @pytest.mark.parametrize("offsets,js", [([1, 2, 5, 18, 20, 33], 3), ([1, 2, 3], 3)])
 def test_parameter_reduction_rule(pkg, device, offsets, js):
     """The parameter sums take one launch up to 32 groups of 64 partial rows and two above.  2048 sequences of one tile
