@@ -178,6 +178,18 @@ def block_backward(dgated, qkvg, pos_bias, scale_embed, phase_base, phase_gain, 
     return (dqkvg, *g[3:7], dgain)
 
 
+class _OnceOnly(torch.autograd.Function):
+    """The gradients as they are, with a graph whose only use is to raise (``anchor``: any tensor with a gradient)."""
+
+    @staticmethod
+    def forward(ctx, anchor, *grads):
+        return grads
+
+    @staticmethod
+    def backward(ctx, *_):
+        raise RuntimeError("the DSQG block has no second derivative")
+
+
 class _DSQGBlockFn(torch.autograd.Function):
     """The block from its input to its output projection as one node (bf16): the two projections, and between them
     the custom ops ``torch.ops.dwarf.dsqg_block_fwd`` / ``dsqg_block_bwd``; the projections' weight and bias
@@ -220,7 +232,11 @@ class _DSQGBlockFn(torch.autograd.Function):
         dqkvg, dpb, dse, dpbase, dpgain, dgain = g
         dwi, dbi = weights(dqkvg, x16, dt_wi, dt_bi, need[1], need[2])
         dx = torch.matmul(dqkvg, wi).to(dt_x) if need[0] else None
-        return (dx, dwi, dbi, dwo, dbo, dpb, dse, dpbase, dpgain, dgain.reshape(gain.shape)) + (None,) * 10
+        grads = (dx, dwi, dbi, dwo, dbo, dpb, dse, dpbase, dpgain, dgain.reshape(gain.shape))
+        if torch.is_grad_enabled() and not torch.compiler.is_compiling():
+            # create_graph: the saved intermediates carry no graph, so a second derivative would lack their terms
+            grads = _OnceOnly.apply(torch.empty(0, device=dy.device, requires_grad=True), *grads)
+        return grads + (None,) * 10
 
 
 def _plain_linear(m) -> bool:

@@ -332,3 +332,21 @@ def test_block_one_node_compiles(pkg, device):
     scale = float(ea.abs().max())
     assert float((ea - eb).abs().max()) <= 2.0 ** -7 * scale
     assert float((a.grad - b.grad).abs().max()) <= 2.0 ** -6 * float(a.grad.abs().max())
+
+
+@pytest.mark.parametrize("inner", ["tables", "nothing"])
+def test_block_second_backward_is_refused(pkg, device, inner):
+    """A gradient taken with create_graph cannot be differentiated again: the second backward raises, also where
+    only the projections and the input have gradients (the tables frozen), and does not give a partial gradient."""
+    offsets = list(pkg.lattice.build_offset_groups(2048)[0])
+    blk = StandInBlock(128, 2, offsets, sum(d <= 28 for d in offsets), 2, 64, seed=6).to(device)
+    if inner == "nothing":
+        for n, p in blk.named_parameters():
+            p.requires_grad_("proj" in n)
+    x = torch.randn(1, 70, 128, generator=torch.Generator().manual_seed(3)).to(device).requires_grad_(True)
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        out = pkg.dsqg_block_forward(blk, x)
+    (dx,) = torch.autograd.grad(out.float().sum(), x, create_graph=True)
+    assert dx.requires_grad
+    with pytest.raises(RuntimeError):
+        (out.float().sum() + dx.square().sum()).backward()
