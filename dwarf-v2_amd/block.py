@@ -240,10 +240,17 @@ class _DSQGBlockFn(torch.autograd.Function):
 
 
 def _plain_linear(m) -> bool:
-    """An nn.Linear nothing hooks into, of whole 16-byte rows: its forward is F.linear on its weight and bias."""
+    """An nn.Linear nothing hooks into, of whole 16-byte rows and plain parameters: its forward is F.linear on its
+    weight and bias.  Hooks of its own, hooks on every module and a forward set on the instance (module trackers,
+    adapters, offloading) need the call, and so does a weight or bias of a class of its own."""
+    every = torch.nn.modules.module
     return (type(m) is torch.nn.Linear and m.in_features % 8 == 0 and m.out_features % 8 == 0
             and not m._forward_pre_hooks and not m._forward_hooks
-            and not m._backward_hooks and not m._backward_pre_hooks)
+            and not m._backward_hooks and not m._backward_pre_hooks
+            and not (every._global_forward_pre_hooks or every._global_forward_hooks
+                     or every._global_backward_hooks or every._global_backward_pre_hooks)
+            and "forward" not in m.__dict__
+            and all(p is None or type(p) in (torch.nn.Parameter, torch.Tensor) for p in (m.weight, m.bias)))
 
 
 def _one_node(block, x: torch.Tensor) -> bool:

@@ -207,3 +207,42 @@ def test_integration_guide_names_exist(pkg):
     assert len(names) >= 15
     missing = [n for n in names if not hasattr(pkg, n)]
     assert not missing, missing
+
+
+# ---- the block's one node: when it runs (no GPU: the block and a stand-in for x on the CPU) --------------------
+def _node_case(pkg, monkeypatch, dtype=torch.bfloat16):
+    from types import SimpleNamespace
+
+    from tests.test_gpu_block import StandInBlock
+
+    monkeypatch.setattr(torch, "is_autocast_enabled", lambda *a: True)
+    monkeypatch.setattr(torch, "get_autocast_dtype", lambda *a: torch.bfloat16)
+    blk = StandInBlock(128, 2, [1, 2, 48, 64], 2, 3, 64, seed=1)
+    x = SimpleNamespace(is_cuda=True, shape=(2, 8, 128), dtype=dtype, device=torch.device("cpu"))
+    assert pkg.block._one_node(blk, SimpleNamespace(**{**vars(x), "dtype": torch.bfloat16}))
+    return blk, x
+
+
+@pytest.mark.parametrize("kind", ["register_module_forward_hook", "register_module_forward_pre_hook",
+                                  "register_module_full_backward_hook", "register_module_full_backward_pre_hook",
+                                  "instance forward", "weight subclass"])
+def test_block_node_gives_way_to_what_changes_a_projection(pkg, monkeypatch, kind):
+    """Hooks on every module, a forward set on the instance and a weight that answers for itself are honoured by
+    calling the projection, so the block is composed then."""
+    blk, x = _node_case(pkg, monkeypatch)
+    if kind.startswith("register"):
+        handle = getattr(torch.nn.modules.module, kind)(lambda *a: None)
+        try:
+            assert not pkg.block._one_node(blk, x)
+        finally:
+            handle.remove()
+        assert pkg.block._one_node(blk, x)
+    elif kind == "instance forward":
+        blk.out_proj.forward = lambda inp: inp
+        assert not pkg.block._one_node(blk, x)
+    else:
+        class Own(torch.Tensor):
+            pass
+
+        blk.qkvg_proj.weight = torch.nn.Parameter(blk.qkvg_proj.weight.detach().as_subclass(Own))
+        assert not pkg.block._one_node(blk, x)
