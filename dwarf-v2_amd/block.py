@@ -45,6 +45,7 @@ from .dsqg import (HEAD_DIM, _check_call, _planes, _rows_ok, _stream, dsqg_atten
 from .npci import npci_rotate
 from .probe import probe_forward
 
+_AUTOCAST_TYPES = (torch.bfloat16, torch.float16, torch.float32)
 NPCI_THETA_MAX = 0.25   # bound of the NPCI rotation angle, theta = 0.25 tanh(raw) (dsqg:71, 3216, 3222)
 
 
@@ -261,7 +262,12 @@ def _one_node(block, x: torch.Tensor) -> bool:
     if torch.is_grad_enabled() and (block.query_probes.requires_grad or block.key_probes.requires_grad):
         return False
     proj, out, D = block.qkvg_proj, block.out_proj, block.num_heads * HEAD_DIM
-    return (_plain_linear(proj) and _plain_linear(out) and block.head_dim == HEAD_DIM
+    if not (_plain_linear(proj) and _plain_linear(out)):
+        return False
+    # what autocast casts; float64 it leaves as it is, for the projections to keep or to refuse
+    if any(t is not None and t.dtype not in _AUTOCAST_TYPES for t in (x, proj.weight, proj.bias, out.weight, out.bias)):
+        return False
+    return (block.head_dim == HEAD_DIM
             and proj.in_features == x.shape[-1] == D and proj.out_features == 4 * D and out.in_features == D
             and proj.weight.device == x.device and out.weight.device == x.device
             and block.if_gain.dtype == torch.float32 and block.if_gain.numel() == block.num_heads

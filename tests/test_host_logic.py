@@ -246,3 +246,15 @@ def test_block_node_gives_way_to_what_changes_a_projection(pkg, monkeypatch, kin
 
         blk.qkvg_proj.weight = torch.nn.Parameter(blk.qkvg_proj.weight.detach().as_subclass(Own))
         assert not pkg.block._one_node(blk, x)
+
+
+@pytest.mark.parametrize("wide", ["x", "qkvg_proj.weight", "qkvg_proj.bias", "out_proj.weight"])
+def test_block_node_leaves_float64_to_the_projections(pkg, monkeypatch, wide):
+    """Autocast leaves float64 alone: a projection of mixed types raises and one all in float64 stays so, which the
+    node, all bf16, would not."""
+    blk, x = _node_case(pkg, monkeypatch, torch.float64 if wide == "x" else torch.float32)
+    if wide != "x":
+        assert pkg.block._one_node(blk, x)
+        p = dict(blk.named_parameters())[wide]
+        p.data = p.data.double()
+    assert not pkg.block._one_node(blk, x)
