@@ -269,7 +269,8 @@ def _one_node(block, x: torch.Tensor) -> bool:
         return False
     return (block.head_dim == HEAD_DIM
             and proj.in_features == x.shape[-1] == D and proj.out_features == 4 * D and out.in_features == D
-            and proj.weight.device == x.device and out.weight.device == x.device
+            and all(t is None or t.device == x.device
+                    for t in (proj.weight, proj.bias, out.weight, out.bias, block.if_gain))
             and block.if_gain.dtype == torch.float32 and block.if_gain.numel() == block.num_heads
             and str(block.backend).lower() in ("auto", "triton", "hip"))
 

@@ -258,3 +258,14 @@ def test_block_node_leaves_float64_to_the_projections(pkg, monkeypatch, wide):
         p = dict(blk.named_parameters())[wide]
         p.data = p.data.double()
     assert not pkg.block._one_node(blk, x)
+
+
+@pytest.mark.parametrize("name", ["if_gain", "qkvg_proj.bias", "out_proj.weight"])
+def test_block_node_only_with_everything_on_one_device(pkg, monkeypatch, name):
+    """The gate's launch reads if_gain by address: a gain elsewhere goes to the composed block, whose product with it
+    raises."""
+    blk, x = _node_case(pkg, monkeypatch)
+    p = dict(blk.named_parameters())[name]
+    owner = blk.get_submodule(name.rpartition(".")[0])
+    setattr(owner, name.rpartition(".")[2], torch.nn.Parameter(torch.empty(p.shape, device="meta")))
+    assert not pkg.block._one_node(blk, x)
