@@ -73,6 +73,20 @@ def _heads(t: torch.Tensor, heads: int) -> torch.Tensor:
     return t.reshape(B, N, heads, D // heads).permute(0, 2, 1, 3)
 
 
+def _expect(ok: bool, what: str) -> None:
+    """The kernels take shapes and types as given: a raw launch on others would read out of range."""
+    if not ok:
+        raise ValueError(f"the raw launch expects {what}")
+
+
+def _check_gate(out, gain, gate, *rows) -> None:
+    B, H, N, hd = out.shape
+    _expect(hd == HEAD_DIM and out.dtype == torch.bfloat16, "out bf16 [B,H,N,64]")
+    _expect(gain.shape == (H,) and gain.dtype == torch.float32 and gain.is_contiguous(), "gain fp32 [H], contiguous")
+    _expect(all(t.shape == (B, N, H * hd) and t.dtype == torch.bfloat16 for t in (gate, *rows)),
+            "gate and its gradients bf16 [B,N,H*64]")
+
+
 def _fill_gate(a: _lib.HeadGateFwdArgs, out, gain, gate) -> None:
     a.B, a.H, a.N = out.shape[:3]
     a.out, a.out_stride = out.data_ptr(), _lib.i64_array(out.stride())
@@ -83,6 +97,7 @@ def _fill_gate(a: _lib.HeadGateFwdArgs, out, gain, gate) -> None:
 def head_gate_forward(out: torch.Tensor, gain: torch.Tensor, gate: torch.Tensor) -> torch.Tensor:
     """Raw launch: bf16((out * gain[h]) * bf16(sigmoid(gate))) as [B,N,H*64]; out bf16 [B,H,N,64], gain fp32
     [H], gate bf16 [B,N,H*64]."""
+    _check_gate(out, gain, gate)
     lib = _lib.load()
     B, H, N, hd = out.shape
     gated = torch.empty((B, N, H * hd), device=out.device, dtype=out.dtype)
@@ -96,6 +111,8 @@ def head_gate_forward(out: torch.Tensor, gain: torch.Tensor, gate: torch.Tensor)
 def head_gate_backward(dgated, out, gain, gate, dgate, *, lse=None, query_start=0, pairs=0):
     """Raw launch: (dout like out, dgain fp32 [H]); the gate's gradient goes into ``dgate``.  pairs: address
     of the [B,H,N] (delta, lse) pairs to write as well, 0 for none."""
+    _check_gate(out, gain, gate, dgated, dgate)
+    _expect(not pairs or (lse.shape == out.shape[:3] and lse.dtype == torch.float32), "lse fp32 [B,H,N] for the pairs")
     lib = _lib.load()
     dout = torch.empty_like(out)
     dgain = torch.empty(gain.shape, device=out.device, dtype=torch.float32)
@@ -118,6 +135,7 @@ def head_gate_backward(dgated, out, gain, gate, dgate, *, lse=None, query_start=
 def linear_wgrad(dy: torch.Tensor, x: torch.Tensor, bias: bool) -> tuple[torch.Tensor, torch.Tensor | None]:
     """Raw launch: (dW [O,I], db [O] or None) fp32 of y = x W^T + b from dy [..., O] and x [..., I] bf16."""
     dy, x = (t.reshape(-1, t.shape[-1]) for t in (dy, x))
+    _expect(dy.shape[0] == x.shape[0] and dy.dtype == x.dtype == torch.bfloat16, "as many bf16 rows of dy as of x")
     dy, x = (t if _rows_ok(t) and t.stride(0) >= t.shape[1] else t.clone(memory_format=torch.contiguous_format)
              for t in (dy, x))
     lib = _lib.load()
@@ -134,10 +152,16 @@ def linear_wgrad(dy: torch.Tensor, x: torch.Tensor, bias: bool) -> tuple[torch.T
     return dw, db
 
 
+def _check_block(qkvg, gain, heads) -> None:
+    _expect(qkvg.dim() == 3 and qkvg.dtype == torch.bfloat16 and qkvg.shape[2] == 4 * HEAD_DIM * heads
+            and gain.shape == (heads,), "qkvg bf16 [B,N,4*64*H] and gain [H]")
+
+
 def block_forward(qkvg, pos_bias, scale_embed, phase_base, phase_gain, query_probes, key_probes, gain, offsets, heads,
                   j_small, j_large, plane_shift, query_start, schedule):
     """Raw launches from the fused projection [B,N,4D] (bf16, contiguous) to the gated heads [B,N,D]: returns
     (gated, out [B,N,H,64], lse, y, z)."""
+    _check_block(qkvg, gain, heads)
     qkvg = qkvg if qkvg.is_contiguous() and _rows_ok(qkvg) else qkvg.clone(memory_format=torch.contiguous_format)
     B, N, D4 = qkvg.shape
     q, k, v, gate = qkvg.split(D4 // 4, dim=-1)
@@ -154,6 +178,11 @@ def block_forward(qkvg, pos_bias, scale_embed, phase_base, phase_gain, query_pro
 def block_backward(dgated, qkvg, pos_bias, scale_embed, phase_base, phase_gain, query_probes, key_probes, gain, offsets,
                    out, lse, y, z, heads, j_small, j_large, plane_shift, query_start, schedule):
     """Raw launches: (dqkvg [B,N,4D], dpos_bias, dscale_embed, dphase_base, dphase_gain, dgain)."""
+    _check_block(qkvg, gain, heads)
+    B, N = qkvg.shape[:2]
+    _expect(out.shape == (B, N, heads, HEAD_DIM) and dgated.shape == (B, N, heads * HEAD_DIM)
+            and lse.shape == (B, heads, N) and y.shape == z.shape == (B, heads, N, 4),
+            "out [B,N,H,64], dgated [B,N,H*64], lse [B,H,N] and y, z [B,H,N,4]")
     qkvg = qkvg if qkvg.is_contiguous() and _rows_ok(qkvg) else qkvg.clone(memory_format=torch.contiguous_format)
     D = qkvg.shape[-1] // 4
     dgated = dgated.to(qkvg.dtype)

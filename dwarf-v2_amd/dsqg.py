@@ -438,6 +438,8 @@ def normalized_probe_banks(query_probes, key_probes, device):
 
 def normalize_probes(query_probes: torch.Tensor, key_probes: torch.Tensor) -> torch.Tensor:
     """Raw launch: [2,4,64] fp32 normalised rows of two fp32 [4,64] banks on one GPU."""
+    if any(p.shape != (R_PLANES, HEAD_DIM) or p.dtype != torch.float32 for p in (query_probes, key_probes)):
+        raise ValueError("the raw launch expects two fp32 [4,64] probe banks")
     qp, kp = query_probes.contiguous(), key_probes.contiguous()
     out = torch.empty((2, R_PLANES, HEAD_DIM), device=qp.device, dtype=torch.float32)
     _lib.check(_lib.load().dwarf_normalize_probes(qp.data_ptr(), kp.data_ptr(), out.data_ptr(), _stream(qp.device)),

@@ -269,3 +269,29 @@ def test_block_node_only_with_everything_on_one_device(pkg, monkeypatch, name):
     owner = blk.get_submodule(name.rpartition(".")[0])
     setattr(owner, name.rpartition(".")[2], torch.nn.Parameter(torch.empty(p.shape, device="meta")))
     assert not pkg.block._one_node(blk, x)
+
+
+def test_block_raw_launches_check_what_their_kernels_assume(pkg):
+    """The raw launches (and the custom ops over them) refuse operands whose shapes or types the kernels would read
+    out of range or as something else, before anything is launched."""
+    b, bf = pkg.block, torch.bfloat16
+    t = lambda *s, dtype=bf: torch.zeros(*s, dtype=dtype)
+    bad = [
+        lambda: b.linear_wgrad(t(4, 8), t(5, 8), True),                       # other row counts
+        lambda: b.linear_wgrad(t(4, 8, dtype=torch.float32), t(4, 8), True),  # not bf16
+        lambda: b.linear_wgrad(t(4, 8), t(4, 8, dtype=torch.float16), True),
+        lambda: b.head_gate_forward(t(1, 2, 4, 64), t(1, dtype=torch.float32), t(1, 4, 128)),
+        lambda: b.head_gate_forward(t(1, 2, 4, 64), t(2), t(1, 4, 128)),
+        lambda: b.head_gate_forward(t(1, 2, 4, 64), t(2, dtype=torch.float32), t(1, 4, 64)),
+        lambda: b.head_gate_forward(t(1, 2, 4, 32), t(2, dtype=torch.float32), t(1, 4, 64)),
+        lambda: b.head_gate_backward(t(1, 4, 64), t(1, 2, 4, 64), t(2, dtype=torch.float32), t(1, 4, 128), t(1, 4, 128)),
+        lambda: b.head_gate_backward(t(1, 4, 128), t(1, 2, 4, 64), t(2, dtype=torch.float32), t(1, 4, 128), t(1, 3, 128)),
+        lambda: b.block_forward(t(1, 4, 256), *[None] * 6, t(2, dtype=torch.float32), None, 2, 1, 1, 0, 1, 0),
+        lambda: b.block_backward(t(1, 4, 128), t(1, 4, 512), *[None] * 6, t(2, dtype=torch.float32), None, t(1, 2, 4, 64),
+                                 *[None] * 3, 2, 1, 1, 0, 1, 0),
+        lambda: pkg.dsqg.normalize_probes(t(3, 64, dtype=torch.float32), t(4, 64, dtype=torch.float32)),
+        lambda: pkg.dsqg.normalize_probes(t(4, 64, dtype=torch.float32), t(4, 64)),
+    ]
+    for i, call in enumerate(bad):
+        with pytest.raises(ValueError, match="expects"):
+            call()
