@@ -45,6 +45,7 @@ from .dsqg import (HEAD_DIM, _check_call, _planes, _rows_ok, _stream, dsqg_atten
 from .npci import npci_rotate
 from .probe import probe_forward
 
+_WGRAD_MAX_STRIDE = 1 << 22
 _AUTOCAST_TYPES = (torch.bfloat16, torch.float16, torch.float32)
 NPCI_THETA_MAX = 0.25   # bound of the NPCI rotation angle, theta = 0.25 tanh(raw) (dsqg:71, 3216, 3222)
 
@@ -136,8 +137,9 @@ def linear_wgrad(dy: torch.Tensor, x: torch.Tensor, bias: bool) -> tuple[torch.T
     """Raw launch: (dW [O,I], db [O] or None) fp32 of y = x W^T + b from dy [..., O] and x [..., I] bf16."""
     dy, x = (t.reshape(-1, t.shape[-1]) for t in (dy, x))
     _expect(dy.shape[0] == x.shape[0] and dy.dtype == x.dtype == torch.bfloat16, "as many bf16 rows of dy as of x")
-    dy, x = (t if _rows_ok(t) and t.stride(0) >= t.shape[1] else t.clone(memory_format=torch.contiguous_format)
-             for t in (dy, x))
+    # the kernel reads a split's rows with 32-bit offsets: rows at most 2^22 elements apart
+    dy, x = (t if _rows_ok(t) and t.shape[1] <= t.stride(0) <= _WGRAD_MAX_STRIDE
+             else t.clone(memory_format=torch.contiguous_format) for t in (dy, x))
     lib = _lib.load()
     dw = torch.empty((dy.shape[1], x.shape[1]), device=dy.device, dtype=torch.float32)
     db = torch.empty(dy.shape[1], device=dy.device, dtype=torch.float32) if bias else None

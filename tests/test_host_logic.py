@@ -295,3 +295,27 @@ def test_block_raw_launches_check_what_their_kernels_assume(pkg):
     for i, call in enumerate(bad):
         with pytest.raises(ValueError, match="expects"):
             call()
+
+
+def test_linear_wgrad_takes_rows_of_any_stride(pkg, monkeypatch):
+    """Rows further apart than the kernel's 32-bit offsets reach (2^22 elements) are copied together first; the
+    library is replaced by a recorder."""
+    b = pkg.block
+    seen = {}
+
+    class Recorder:
+        def dwarf_linear_wgrad_workspace_bytes(self, args):
+            return 0
+
+        def dwarf_linear_wgrad(self, args, stream):
+            seen.update(dy=args._obj.dy_stride, x=args._obj.x_stride)
+            return 0
+
+    monkeypatch.setattr(b._lib, "load", lambda: Recorder())
+    monkeypatch.setattr(b, "_stream", lambda device: 0)
+    far = torch.zeros(2, (1 << 22) + 8, dtype=torch.bfloat16)
+    b.linear_wgrad(far[:, :16], far[:, :8], True)
+    assert seen == {"dy": 16, "x": 8}
+    near = torch.zeros(2, 1 << 22, dtype=torch.bfloat16)
+    b.linear_wgrad(near[:, :16], near[:, :8], True)
+    assert seen == {"dy": 1 << 22, "x": 1 << 22}
