@@ -24,6 +24,16 @@ __device__ __forceinline__ uint4 pack8(const float* x) {
 }
 __device__ __forceinline__ float sigmoid_bf16(float x) { return round_bf16(__fdividef(1.f, 1.f + __expf(-x))); }
 
+// <y, o> over the item's 64 dims in every lane, in the order of the DSQG backward's own delta (dsqg_bwd_dq.hip: 16
+// dims to a lane as one chain, then four lanes), so both give the same bits: lane 2g + 1 goes on with lane 2g's chain.
+__device__ __forceinline__ float item_delta(const uint4& y, const uint4& o) {
+  auto chain = [&](float x) { return dot2bf(y.w, o.w, dot2bf(y.z, o.z, dot2bf(y.y, o.y, dot2bf(y.x, o.x, x)))); };
+  float x = chain(dpp_f<0xA0>(chain(0.f)));   // quad_perm [0,0,2,2]
+  x = dpp_f<0xF5>(x);                         // quad_perm [1,1,3,3]: lanes 2g and 2g + 1 hold slice g
+  x += dpp_f<0x4E>(x);                        // slices 0 + 1 and 2 + 3
+  return x + dpp_f<0x141>(x);                 // row_half_mirror: lane i of eight <-> 7 - i
+}
+
 // Sum over the item's eight lanes, in every lane.
 __device__ __forceinline__ float item_sum(float x) {
   x = group_sum<4>(x);
@@ -102,8 +112,7 @@ __global__ __launch_bounds__(kBlock) void head_gate_bwd_kernel(const dwarf_head_
         pack8(x);
     if (a.delta_pairs) {
       const bool mass = static_cast<int>(t.n) >= a.query_start && lse > -INFINITY;
-      float dlt = dot2bf(yw.w, ow.w, dot2bf(yw.z, ow.z, dot2bf(yw.y, ow.y, dot2bf(yw.x, ow.x, 0.f))));
-      dlt = item_sum(dlt);
+      const float dlt = item_delta(yw, ow);
       if (c == 0)
         *reinterpret_cast<float2*>(a.delta_pairs + 2 * ((static_cast<int64_t>(t.b) * f.H + t.h) * f.N + t.n)) =
             make_float2(dlt, mass ? lse * kLog2e : INFINITY);

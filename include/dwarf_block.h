@@ -69,8 +69,10 @@ int dwarf_head_gate_fwd(const dwarf_head_gate_fwd_args* args, dwarf_stream_t str
  * dgain[h] = sum of dm * out in fp32 in a fixed order.  fwd.gated is not used.
  *
  * delta_pairs (may be NULL): [B,H,N] pairs (sum_d dout * out, lse * log2 e; +inf where lse is -inf or
- * n < query_start), what dwarf_dsqg_bwd_delta writes at the start of the DSQG backward's workspace; a caller
- * that passes the workspace's address here runs its stages under DWARF_SCHED_DELTA_STAGE without that launch.
+ * n < query_start), what dwarf_dsqg_bwd_delta writes at the start of the DSQG backward's workspace, summed in
+ * its order and so with its bits (before query_start it writes 0, which is this sum over the zero rows of out);
+ * a caller that passes the workspace's address here runs its stages under DWARF_SCHED_DELTA_STAGE without that
+ * launch.
  * lse [B,H,N] fp32 is read then.
  */
 typedef struct {

@@ -350,3 +350,23 @@ def test_block_second_backward_is_refused(pkg, device, inner):
     assert dx.requires_grad
     with pytest.raises(RuntimeError):
         (out.float().sum() + dx.square().sum()).backward()
+
+
+@pytest.mark.parametrize("H,N,lattice", [(8, 1025, "canonical"), (3, 700, "far")])
+def test_block_schedules_give_the_same_bits(pkg, device, monkeypatch, H, N, lattice):
+    """The block's backward with the gate launch's (delta, lse) pairs beside two streams, and with one stream, where
+    the dQ launch forms them: every gradient bit for bit.  "far": queries before the smallest offset take no part."""
+    offsets, js = (list(pkg.ALL_OFFSETS), 17) if lattice == "canonical" else ([64, 96, 128, 200, 333], 0)
+    blk = StandInBlock(64 * H, H, offsets, js, 3, 10 ** 6, seed=17).to(device)   # 10^6: no support cropping
+    g = torch.Generator().manual_seed(18)
+    x = torch.randn(2, N, 64 * H, generator=g).to(torch.bfloat16).to(device).requires_grad_(True)
+    dy = torch.randn(2, N, 64 * H, generator=g).to(torch.bfloat16).to(device)
+    params = [p for n, p in blk.named_parameters() if p.requires_grad and not n.startswith("npci")]
+    got = {}
+    for two in (True, False):
+        monkeypatch.setattr(pkg.dsqg, "_worth_two_streams", lambda q, J: two)
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            out = pkg.dsqg_block_forward(blk, x)
+        got[two] = torch.autograd.grad(out, [x] + params, dy)
+    for i, (a, b) in enumerate(zip(got[True], got[False])):
+        assert torch.equal(a, b), i
