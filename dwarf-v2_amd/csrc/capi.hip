@@ -790,7 +790,7 @@ int dwarf_linear_wgrad(const dwarf_linear_wgrad_args* args, dwarf_stream_t strea
   if (a.dy_stride < a.O || a.x_stride < a.I || a.dy_stride > (1 << 22) || a.x_stride > (1 << 22))
     return fail(DWARF_ERR_UNSUPPORTED, "row strides must lie between the row length and 2^22 elements");
   const size_t need = dwarf::linear_wgrad_workspace(a);
-  if (!a.workspace || a.workspace_bytes < need || !aligned16(a.workspace))
+  if (need > 0 && (!a.workspace || a.workspace_bytes < need || !aligned16(a.workspace)))
     return fail(DWARF_ERR_WORKSPACE, "workspace needs %zu bytes, 16-byte aligned, got %zu", need, a.workspace_bytes);
   return hip_status(dwarf::launch_linear_wgrad(a, s), "dwarf_linear_wgrad");
 }

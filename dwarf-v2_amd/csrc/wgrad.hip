@@ -19,6 +19,12 @@
 // four waves of 64 x 128 107 and 42 (nothing to issue while a wave waits for
 // its operands), two workgroups of 128 x 128 per CU 107 and 43, the bias as
 // dot products of the operands 100 and 38.
+// One split (more than 128 tiles, or at most four 64-row steps) writes dW and
+// db itself instead of a partial and a copy of it: 16,384 x 4,096 from 256
+// rows 204 -> 89 us, 8,192 x 2,048 from 200, 2,048 and 8,192 rows 52 -> 32,
+// 117 -> 97, 346 -> 312 (the library, to bf16, with the cast and the bias:
+// 141, 53, 116, 297; it is ahead from there on, 1,142 against 972 at 30,720
+// rows, and rounds dW to bf16).
 #include "common.h"
 #include "dsqg_internal.h"
 #include "dwarf_block.h"
@@ -220,18 +226,21 @@ WgradPlan wgrad_plan(const dwarf_linear_wgrad_args& a) {
 
 }  // namespace
 
+// One split writes dW and db itself: no partials, no second launch.
 size_t linear_wgrad_workspace(const dwarf_linear_wgrad_args& a) {
   const WgradPlan p = wgrad_plan(a);
+  if (p.splits == 1) return 0;
   return static_cast<size_t>(p.splits) * (static_cast<size_t>(a.O) * a.I + a.O) * sizeof(float);
 }
 
 hipError_t launch_linear_wgrad(const dwarf_linear_wgrad_args& a, hipStream_t stream) {
   const WgradPlan p = wgrad_plan(a);
   const int64_t n = static_cast<int64_t>(a.O) * a.I;
-  float* part = static_cast<float*>(a.workspace);
-  float* part_b = part + p.splits * n;
+  float* part = p.splits > 1 ? static_cast<float*>(a.workspace) : a.dw;
+  float* part_b = p.splits > 1 ? part + p.splits * n : a.db;
   hipLaunchKernelGGL(linear_wgrad_kernel, dim3(p.tiles_o * p.tiles_i * p.splits), dim3(kWgThreads), 2 * kStageBytes, stream, a,
                      p.splits, p.rows_per, p.tiles_i, part, part_b);
+  if (p.splits == 1) return hipGetLastError();
   const int64_t quads = (n + (a.db ? a.O : 0)) / 4;
   hipLaunchKernelGGL(linear_wgrad_sum, dim3(static_cast<unsigned>((quads + kBlock - 1) / kBlock)), dim3(kBlock), 0, stream,
                      part, part_b, p.splits, n, a.db ? static_cast<int64_t>(a.O) : 0, a.dw, a.db);

@@ -373,3 +373,15 @@ def test_block_entries_refuse_bad_calls_without_gpu(pkg, lib):
     w.I, w.x_stride = 512, 504
     assert lib.dwarf_linear_wgrad(ctypes.byref(w), None) == L.DWARF_ERR_UNSUPPORTED   # rows that overlap
     assert lib.dwarf_linear_wgrad(None, None) == bad
+
+
+def test_linear_wgrad_of_one_split_needs_no_workspace(pkg, lib):
+    """Where the output tiles or the few rows leave one split, dW and db are written by the product's launch itself:
+    no partial as large as dW."""
+    L = pkg._lib
+    w = L.LinearWgradArgs()
+    for M, O, I in ((200, 2048, 512), (8192, 8192, 2048), (1, 8, 8)):
+        w.M, w.O, w.I, w.dy_stride, w.x_stride = M, O, I, O, I
+        assert lib.dwarf_linear_wgrad_workspace_bytes(ctypes.byref(w)) == 0, (M, O, I)
+    w.M, w.O, w.I, w.dy_stride, w.x_stride = 30720, 2048, 2048, 2048, 2048   # 128 tiles, 2 splits
+    assert lib.dwarf_linear_wgrad_workspace_bytes(ctypes.byref(w)) == 2 * (2048 * 2048 + 2048) * 4
