@@ -13,7 +13,7 @@ from ctypes import POINTER, c_char_p, c_float, c_int, c_int32, c_int64, c_size_t
 
 LIB_NAME = "libdwarf_dsqg.so"
 LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), LIB_NAME)
-ABI_VERSION = 9
+ABI_VERSION = 10
 
 DWARF_OK = 0
 DWARF_ERR_INVALID_ARGUMENT = 1
@@ -341,6 +341,10 @@ def load() -> ctypes.CDLL:
     lib = ctypes.CDLL(LIB_PATH)
     lib.dwarf_abi_version.restype = c_int
     lib.dwarf_abi_version.argtypes = []
+    # before any other symbol: a library of another version may lack some
+    version = lib.dwarf_abi_version()
+    if version != ABI_VERSION:
+        raise NativeLibraryError(f"{LIB_NAME} ABI {version} does not match the binding's ABI {ABI_VERSION}")
     lib.dwarf_last_error.restype = c_char_p
     lib.dwarf_last_error.argtypes = []
     lib.dwarf_dsqg_fwd.restype = c_int
@@ -422,9 +426,6 @@ def load() -> ctypes.CDLL:
     lib.dwarf_head_gate_bwd_workspace_bytes.argtypes = [POINTER(HeadGateBwdArgs)]
     lib.dwarf_head_gate_bwd.restype = c_int
     lib.dwarf_head_gate_bwd.argtypes = [POINTER(HeadGateBwdArgs), c_void_p]
-    version = lib.dwarf_abi_version()
-    if version != ABI_VERSION:
-        raise NativeLibraryError(f"{LIB_NAME} ABI {version} does not match the binding's ABI {ABI_VERSION}")
     _LIB = lib
     return lib
 

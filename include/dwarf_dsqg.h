@@ -25,7 +25,7 @@
 extern "C" {
 #endif
 
-#define DWARF_ABI_VERSION 9
+#define DWARF_ABI_VERSION 10
 #define DWARF_R_PLANES 4        /* MOVT planes per far offset: dsqg:69 */
 #define DWARF_Q6_GROUP 32       /* head-dim elements per q6 scale group */
 #define DWARF_Q6_SLOT_BYTES 128 /* one q6 K/V cache slot per (b, kv head, t) */

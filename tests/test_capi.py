@@ -385,3 +385,16 @@ def test_linear_wgrad_of_one_split_needs_no_workspace(pkg, lib):
         assert lib.dwarf_linear_wgrad_workspace_bytes(ctypes.byref(w)) == 0, (M, O, I)
     w.M, w.O, w.I, w.dy_stride, w.x_stride = 30720, 2048, 2048, 2048, 2048   # 128 tiles, 2 splits
     assert lib.dwarf_linear_wgrad_workspace_bytes(ctypes.byref(w)) == 2 * (2048 * 2048 + 2048) * 4
+
+
+@pytest.mark.skipif(shutil.which("gcc") is None, reason="gcc not available")
+def test_a_library_of_another_abi_is_named_as_such(pkg, tmp_path, monkeypatch):
+    """A library built before the newest entry points says so by its ABI number, and not by a missing symbol."""
+    L = pkg._lib
+    src, so = tmp_path / "old.c", tmp_path / "libold.so"
+    src.write_text("int dwarf_abi_version(void) { return 9; }\n")
+    subprocess.run(["gcc", "-shared", "-fPIC", str(src), "-o", str(so)], check=True)
+    monkeypatch.setattr(L, "_LIB", None)
+    monkeypatch.setattr(L, "LIB_PATH", str(so))
+    with pytest.raises(L.NativeLibraryError, match="ABI 9"):
+        L.load()
