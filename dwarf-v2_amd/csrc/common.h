@@ -41,57 +41,23 @@ __device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {
 // 16-byte vector loads and widened to fp32, or narrowed and stored.
 // ---------------------------------------------------------------------------
 template <typename T, int CNT>
-__device__ __forceinline__ void load_f32(const T* __restrict__ p, float* __restrict__ dst);
-
-template <int CNT>
-__device__ __forceinline__ void load_f32_bf16(const uint16_t* __restrict__ p, float* __restrict__ dst) {
-  static_assert(CNT % 8 == 0, "chunk must be whole 16-byte vectors");
+__device__ __forceinline__ void load_f32(const T* __restrict__ p, float* __restrict__ dst) {
+  constexpr int kPer = 16 / sizeof(T);
+  static_assert(CNT % kPer == 0, "chunk must be whole 16-byte vectors");
   const uint4* v = reinterpret_cast<const uint4*>(p);
 #pragma unroll
-  for (int i = 0; i < CNT / 8; ++i) {
+  for (int i = 0; i < CNT / kPer; ++i) {
     const uint4 w = v[i];
-    dst[8 * i + 0] = bf16_lo(w.x); dst[8 * i + 1] = bf16_hi(w.x);
-    dst[8 * i + 2] = bf16_lo(w.y); dst[8 * i + 3] = bf16_hi(w.y);
-    dst[8 * i + 4] = bf16_lo(w.z); dst[8 * i + 5] = bf16_hi(w.z);
-    dst[8 * i + 6] = bf16_lo(w.w); dst[8 * i + 7] = bf16_hi(w.w);
+    float* d = dst + kPer * i;
+    if constexpr (sizeof(T) == 2) {
+      d[0] = bf16_lo(w.x); d[1] = bf16_hi(w.x); d[2] = bf16_lo(w.y); d[3] = bf16_hi(w.y);
+      d[4] = bf16_lo(w.z); d[5] = bf16_hi(w.z); d[6] = bf16_lo(w.w); d[7] = bf16_hi(w.w);
+    } else {
+      d[0] = __uint_as_float(w.x); d[1] = __uint_as_float(w.y);
+      d[2] = __uint_as_float(w.z); d[3] = __uint_as_float(w.w);
+    }
   }
 }
-
-template <>
-__device__ __forceinline__ void load_f32<bf16, 64>(const bf16* p, float* dst) {
-  load_f32_bf16<64>(reinterpret_cast<const uint16_t*>(p), dst);
-}
-template <>
-__device__ __forceinline__ void load_f32<bf16, 32>(const bf16* p, float* dst) {
-  load_f32_bf16<32>(reinterpret_cast<const uint16_t*>(p), dst);
-}
-template <>
-__device__ __forceinline__ void load_f32<bf16, 16>(const bf16* p, float* dst) {
-  load_f32_bf16<16>(reinterpret_cast<const uint16_t*>(p), dst);
-}
-template <>
-__device__ __forceinline__ void load_f32<bf16, 8>(const bf16* p, float* dst) {
-  load_f32_bf16<8>(reinterpret_cast<const uint16_t*>(p), dst);
-}
-
-template <int CNT>
-__device__ __forceinline__ void load_f32_f32(const float* __restrict__ p, float* __restrict__ dst) {
-  static_assert(CNT % 4 == 0, "chunk must be whole 16-byte vectors");
-  const float4* v = reinterpret_cast<const float4*>(p);
-#pragma unroll
-  for (int i = 0; i < CNT / 4; ++i) {
-    const float4 w = v[i];
-    dst[4 * i + 0] = w.x; dst[4 * i + 1] = w.y; dst[4 * i + 2] = w.z; dst[4 * i + 3] = w.w;
-  }
-}
-template <>
-__device__ __forceinline__ void load_f32<float, 64>(const float* p, float* dst) { load_f32_f32<64>(p, dst); }
-template <>
-__device__ __forceinline__ void load_f32<float, 32>(const float* p, float* dst) { load_f32_f32<32>(p, dst); }
-template <>
-__device__ __forceinline__ void load_f32<float, 16>(const float* p, float* dst) { load_f32_f32<16>(p, dst); }
-template <>
-__device__ __forceinline__ void load_f32<float, 8>(const float* p, float* dst) { load_f32_f32<8>(p, dst); }
 
 // 16 consecutive values as raw 16-byte vectors, so that a later step's row
 // can be requested before the current one is used (software prefetch).
@@ -124,9 +90,6 @@ __device__ __forceinline__ void widen(const RawSlice16<float>& r, float* x) {
   }
 }
 
-template <typename T, int CNT>
-__device__ __forceinline__ void store_from_f32(T* __restrict__ p, const float* __restrict__ src);
-
 template <int CNT>
 __device__ __forceinline__ void store_bf16(uint16_t* __restrict__ p, const float* __restrict__ src) {
   uint4* v = reinterpret_cast<uint4*>(p);
@@ -140,14 +103,6 @@ __device__ __forceinline__ void store_bf16(uint16_t* __restrict__ p, const float
     v[i] = w;
   }
 }
-template <>
-__device__ __forceinline__ void store_from_f32<bf16, 64>(bf16* p, const float* src) {
-  store_bf16<64>(reinterpret_cast<uint16_t*>(p), src);
-}
-template <>
-__device__ __forceinline__ void store_from_f32<bf16, 32>(bf16* p, const float* src) {
-  store_bf16<32>(reinterpret_cast<uint16_t*>(p), src);
-}
 
 template <int CNT>
 __device__ __forceinline__ void store_f32(float* __restrict__ p, const float* __restrict__ src) {
@@ -155,34 +110,12 @@ __device__ __forceinline__ void store_f32(float* __restrict__ p, const float* __
 #pragma unroll
   for (int i = 0; i < CNT / 4; ++i) v[i] = make_float4(src[4 * i], src[4 * i + 1], src[4 * i + 2], src[4 * i + 3]);
 }
-template <>
-__device__ __forceinline__ void store_from_f32<float, 64>(float* p, const float* src) { store_f32<64>(p, src); }
-template <>
-__device__ __forceinline__ void store_from_f32<float, 32>(float* p, const float* src) { store_f32<32>(p, src); }
 
-// ---------------------------------------------------------------------------
-// Math.  FAST selects the hardware transcendental instructions (bf16 paths,
-// where results are rounded to bf16 anyway); otherwise the correctly
-// range-reduced device-library routines are called (fp32 parity paths).
-// ---------------------------------------------------------------------------
-template <bool FAST>
-__device__ __forceinline__ float dexp(float x) {
-  if constexpr (FAST) return __expf(x);
-  else return expf(x);
-}
-template <bool FAST>
-__device__ __forceinline__ float dlog(float x) {
-  if constexpr (FAST) return __logf(x);
-  else return logf(x);
-}
-template <bool FAST>
+// Sine and cosine by the hardware's instructions (the bf16 kernels, whose results are rounded to bf16 anyway; the fp32
+// kernels call the device library's range-reduced routines).
 __device__ __forceinline__ void dsincos(float x, float* s, float* c) {
-  if constexpr (FAST) {
-    *s = __sinf(x);
-    *c = __cosf(x);
-  } else {
-    sincosf(x, s, c);
-  }
+  *s = __sinf(x);
+  *c = __cosf(x);
 }
 
 // ---------------------------------------------------------------------------

@@ -269,7 +269,7 @@ __global__ __launch_bounds__(kBlock, MINWG) void dsqg_bwd_dkdv_bf16_k4(const dwa
         if (far) {
           const float2 ph = ph_h[(j - J_small) * kPlanes + g];
           pg = ph.y;
-          dsincos<true>(fmaf(ph.y * c.y[jj], zg, ph.x), &sn, &cs);
+          dsincos(fmaf(ph.y * c.y[jj], zg, ph.x), &sn, &cs);
           gd += da * (cs * va - sn * vb - va) + db * (sn * va + cs * vb - vb);
         }
         dot = group_sum<4>(dot);

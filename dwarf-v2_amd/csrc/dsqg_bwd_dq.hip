@@ -452,7 +452,7 @@ __global__ __launch_bounds__(kBlock, kGatherWgsPerCu) void dsqg_bwd_dq_bf16_g4(
           const float2 ph = s_ph[(j - J_small) * kPlanes + g];
           pg = ph.y;
           float sn, cs;
-          dsincos<true>(fmaf(ph.y * yg, c.z[jj], ph.x), &sn, &cs);
+          dsincos(fmaf(ph.y * yg, c.z[jj], ph.x), &sn, &cs);
           const float va = (SHIFT & 1) ? bf16_hi(vw[SHIFT >> 1]) : bf16_lo(vw[SHIFT >> 1]);
           const float vb = ((SHIFT + 1) & 1) ? bf16_hi(vw[(SHIFT + 1) >> 1]) : bf16_lo(vw[(SHIFT + 1) >> 1]);
           const float da = (SHIFT & 1) ? bf16_hi(d32[SHIFT >> 1]) : bf16_lo(d32[SHIFT >> 1]);

@@ -253,7 +253,7 @@ __global__ __launch_bounds__(kBlock, 2) void dsqg_fwd_bf16_q4(const dwarf_dsqg_f
       if (j >= J_small && j < J) {
         const float2 ph = s_ph[(j - J_small) * kPlanes + g];
         float sn, cs;
-        dsincos<true>(fmaf(ph.y * yg, c.z[jj], ph.x), &sn, &cs);
+        dsincos(fmaf(ph.y * yg, c.z[jj], ph.x), &sn, &cs);
         const float va = vf[SHIFT], vb = vf[SHIFT + 1];
         vf[SHIFT] = cs * va - sn * vb;
         vf[SHIFT + 1] = sn * va + cs * vb;
@@ -535,7 +535,7 @@ __global__ __launch_bounds__(kBlock, 2) void dsqg_fwd_bf16_win(const dwarf_dsqg_
       if (j >= J_small && j < J) {
         const float2 ph = s_ph[(j - J_small) * kPlanes + g];
         float sn, cs;
-        dsincos<true>(fmaf(ph.y * yg, c.z[jj], ph.x), &sn, &cs);
+        dsincos(fmaf(ph.y * yg, c.z[jj], ph.x), &sn, &cs);
         const float va = vf[SHIFT], vb = vf[SHIFT + 1];
         vf[SHIFT] = cs * va - sn * vb;
         vf[SHIFT + 1] = sn * va + cs * vb;

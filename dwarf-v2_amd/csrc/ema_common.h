@@ -111,7 +111,6 @@ constexpr int kRows = sizeof(T) == 2 ? 16 : 8;
 // end state does not depend on the state entering it.
 constexpr int kCarryWaves = 16;
 constexpr int kCarryChannels = 16;
-constexpr int kCarrySegs = kCarryWaves * (kWave / kCarryChannels);
 constexpr int kCarrySeg = 32;   // chunk states a lane holds in registers per pass
 constexpr int kDaRows = 16;     // dalpha partials loaded per block
 

@@ -60,6 +60,4 @@ __device__ __forceinline__ void split_bf16x8(const float* x, bf16x8& hi, bf16x8&
 
 __device__ __forceinline__ bf16x8 bf16x8_from_bits(uint4 w) { return __builtin_bit_cast(bf16x8, w); }
 
-__device__ __forceinline__ bf16x8 bf16x8_zero() { return __builtin_bit_cast(bf16x8, uint4{0u, 0u, 0u, 0u}); }
-
 }  // namespace dwarf

@@ -641,7 +641,7 @@ __global__ __launch_bounds__(kBlock, 2) void q6_prefill_q4(const dwarf_dsqg_q6_p
     if (s.j >= J_small && s.j < J) {   // wave-uniform
       const float2 ph = s_ph[(s.j - J_small) * kPlanes + g];
       float sn, cs;
-      dsincos<true>(fmaf(ph.y * yg, zf, ph.x), &sn, &cs);
+      dsincos(fmaf(ph.y * yg, zf, ph.x), &sn, &cs);
       const float va = cf[SHIFT], vb = cf[SHIFT + 1];
       cf[SHIFT] = cs * va - sn * vb;
       cf[SHIFT + 1] = sn * va + cs * vb;
@@ -943,7 +943,7 @@ __global__ __launch_bounds__(kBlock, 2) void q6_prefill_win(const dwarf_dsqg_q6_
       if (s.j >= J_small && s.j < J) {   // wave-uniform
         const float2 ph = s_ph[(s.j - J_small) * kPlanes + g];
         float sn, cs;
-        dsincos<true>(fmaf(ph.y * yg, zf, ph.x), &sn, &cs);
+        dsincos(fmaf(ph.y * yg, zf, ph.x), &sn, &cs);
         const float va = cf[SHIFT], vb = cf[SHIFT + 1];
         cf[SHIFT] = cs * va - sn * vb;
         cf[SHIFT + 1] = sn * va + cs * vb;
@@ -1446,7 +1446,7 @@ __global__ __launch_bounds__(kWave * kMaxDecHeads) void q6_decode_q4(const dwarf
     // has no far row.
     if (uniform(list[k0 + kDecRows - 1].x) >= J_small) {
       float sn, cs;
-      dsincos<true>(fmaf(b.gain * yg, b.z, b.base), &sn, &cs);
+      dsincos(fmaf(b.gain * yg, b.z, b.base), &sn, &cs);
       const float va = cf[SHIFT], vb = cf[SHIFT + 1];
       cf[SHIFT] = cs * va - sn * vb;
       cf[SHIFT + 1] = sn * va + cs * vb;
