@@ -315,7 +315,7 @@ def test_block_node_with_frozen_parts(pkg, device, frozen):
 
 
 def test_block_one_node_compiles(pkg, device):
-    """torch.compile traces the block's node with fullgraph and gives the eager bits."""
+    """torch.compile traces the block's node with fullgraph; out and dx have the eager bits (the same launches)."""
     offsets = list(pkg.lattice.build_offset_groups(2048)[0])
     blk = StandInBlock(256, 4, offsets, sum(d <= 28 for d in offsets), 2, 64, seed=3).to(device)
     x = torch.randn(2, 96, 256, generator=torch.Generator().manual_seed(1)).to(torch.bfloat16).to(device)
@@ -329,9 +329,7 @@ def test_block_one_node_compiles(pkg, device):
     eb = torch.compile(step, fullgraph=True)(b)
     ea.float().sum().backward()
     eb.float().sum().backward()
-    scale = float(ea.abs().max())
-    assert float((ea - eb).abs().max()) <= 2.0 ** -7 * scale
-    assert float((a.grad - b.grad).abs().max()) <= 2.0 ** -6 * float(a.grad.abs().max())
+    assert torch.equal(ea, eb) and torch.equal(a.grad, b.grad)
 
 
 @pytest.mark.parametrize("inner", ["tables", "nothing"])

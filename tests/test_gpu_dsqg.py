@@ -297,10 +297,15 @@ def test_two_stream_backward_leaves_nothing_in_use(pkg, device, B, h, N):
                 assert torch.equal(a, b)
 
 
-@pytest.mark.parametrize("near", [6, 7, 10, 11])
-def test_default_schedule_by_near_offsets(pkg, device, near):
+@pytest.mark.parametrize("below", [1, 0])
+@pytest.mark.parametrize("rule", ["BAND_MIN_FORWARD", "BAND_MIN_BACKWARD"])
+def test_default_schedule_by_near_offsets(pkg, device, rule, below):
     """The baseline mode on either side of the counts at which the forward and the backward turn from the gather
-    loops to the near band (a forward with the band and a backward without in between), against the oracle."""
+    loops to the near band (both gathered, a forward with the band beside a gathered backward, both with the band),
+    against the oracle."""
+    near = getattr(pkg.dsqg, rule) - below
+    taken = [pkg.dsqg.schedule_for(0, True, near, back) for back in (False, True)]
+    assert taken[rule == "BAND_MIN_BACKWARD"] == (0 if below else pkg._lib.DWARF_SCHED_BAND)
     full = lattice(pkg)
     offsets = full[17 - near:17] + full[17:40]
     x = make_inputs(1, 3, 3, 530, offsets, near, seed=200 + near, dtype=torch.bfloat16, plane_shift=3, gain_std=4.0)
