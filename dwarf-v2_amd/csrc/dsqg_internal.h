@@ -42,7 +42,8 @@ struct BwdWorkspace {
   size_t part_se_off, part_se_bytes;    // [W][J][64] fp32
   size_t part_pb_off, part_pb_bytes;    // [H][pb_rows][J] fp32
   size_t part_ph_off, part_ph_bytes;    // [H][ph_rows][J_L][8] fp32
-  size_t ds_off, ds_bytes;              // bf16: dS [B*H][J][N] fp32; fp32: dS, then P, [B*H][J][np]
+  size_t ds_off, ds_bytes;              // bf16: dS [B*H][J][N] fp32; fp32: dS, then P, [B*H][J][np] (189 MB at
+                                        // B15 H8 N2048 J96, 755 MB at N8192)
   size_t red_off, red_bytes;            // stage-1 sums of the reduction
   size_t kv_part_off, kv_part_bytes;    // bf16, kv_split > 1: [kv_split][split units x 64 keys] partial dK and
                                         // dV (64 fp32 each), then dZ (4 fp32), of each subset of the query heads

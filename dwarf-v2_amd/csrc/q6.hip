@@ -1130,7 +1130,9 @@ constexpr int kDecSplitWaves = 4;     // waves that share a head's list in the s
 // heads, 96 offsets, device time against the table's two launches: 1 sequence
 // 4.7 / 11.5 us, 5 5.4 / 11.7, 14 7.1 / 12.0, 28 (2016 items) 11.2 / 13.2, 42
 // (3024) 15.8 / 14.9, 128 41 / 25.5; 28 sequences of 300 tokens 10.3 / 11.9, of
-// 2048 with two KV heads 12.1 / 14.2.
+// 2048 with two KV heads 12.1 / 14.2.  With 256 offsets, per graph replay (a
+// replay of anything takes 17): 1 sequence 17 / 27, 5 17 / 28, 14 20 / 29, 28
+// 29 / 36; the line holds for the longest list too.
 constexpr int kDecSplitItems = 2048;
 
 struct DecBatch {
@@ -1277,8 +1279,8 @@ __device__ __forceinline__ float wave_allsum(float x) { return sum_over_queries1
 // table launch, then a wave's six batches.  Here a workgroup's four waves share
 // one head's list, wave w taking batches w, w + 4, ..., and each row's
 // <q, e_j> is formed beside its q.k from the E row (bf16, hi and lo for the
-// fp32 table), so there is no table launch and at most two batches in turn;
-// the waves join through LDS.  For many items that costs more than the table
+// fp32 table), so there is no table launch and two batches in turn at 96
+// offsets (four at 256); the waves join through LDS.  For many items that costs more than the table
 // (eight v_dot2, eight conversions and four loads a row).
 template <int SHIFT, bool SPLIT>
 __global__ __launch_bounds__(kWave * kMaxDecHeads) void q6_decode_q4(const dwarf_dsqg_q6_decode_args a,

@@ -64,9 +64,10 @@ typedef struct {
 int dwarf_head_gate_fwd(const dwarf_head_gate_fwd_args* args, dwarf_stream_t stream);
 
 /*
- * The gradients autograd forms for that expression, with its roundings: with s = bf16(sigmoid(gate)) and
- * dm = dgated * s, dout = bf16(dm * gain), dgate = bf16(bf16(dgated * out * gain) * (1 - s) * s) and
- * dgain[h] = sum of dm * out in fp32 in a fixed order.  fwd.gated is not used.
+ * The gradients of that expression: with s = bf16(sigmoid(gate)) and dm = dgated * s, dout = bf16(dm * gain),
+ * dgate = bf16(bf16(dgated * out * gain) * (1 - s) * s) and dgain[h] = sum of dm * out in fp32 in a fixed
+ * order, rounded where autograd rounds them but for dgate, whose last product autograd forms from
+ * bf16(bf16(...) * (1 - s)).  fwd.gated is not used.
  *
  * delta_pairs (may be NULL): [B,H,N] pairs (sum_d dout * out, lse * log2 e; +inf where lse is -inf or
  * n < query_start), what dwarf_dsqg_bwd_delta writes at the start of the DSQG backward's workspace, summed in
