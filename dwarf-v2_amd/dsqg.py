@@ -38,8 +38,9 @@ DEFAULT_SCHEDULE = _lib.DWARF_SCHED_BAND
 # Fewest near offsets that go to the band.  Band against gather in us, overlapped backward: B15 T2048, 23 far: 6 near
 # 269 / 239, 9 273 / 255, 10 271 / 263, 12 271 / 273, 17 278 / 305; 79 far: 9 454 / 438, 10 450 / 450, 12 454 / 461;
 # B4 T8192, 23 far: 9 354 / 336, 10 351 / 352, 12 355 / 361.  Forward, B15 T2048, 23 far: 3 near 71 / 62, 6 68 / 67,
-# 8 70 / 73, 10 69 / 78; B4 T8192, 79 far: 6 208 / 209, 8 210 / 210, 10 207 / 214.  At 6 the two are even there, and two
-# other forwards with 6 near and 23 far were faster on the band (52 / 53, 80 / 82), so 6 is the band's.
+# 8 70 / 73, 10 69 / 78; B4 T8192, 79 far: 6 208 / 209, 8 210 / 210, 10 207 / 214.  At 6 near and 23 far the two are
+# even with y given (B15 T2048 66.8 / 66.2, B4 T8192 85.7 / 86.0, B7 T1999 38.7 / 37.2) and the band is ahead with y
+# formed in the kernel, the block's form (74.9 / 76.4, 94.7 / 96.1, 42.3 / 42.5), so 6 is the band's.
 BAND_MIN_FORWARD, BAND_MIN_BACKWARD = 6, 11
 
 
