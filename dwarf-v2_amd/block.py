@@ -103,6 +103,10 @@ def head_gate_forward(out: torch.Tensor, gain: torch.Tensor, gate: torch.Tensor)
     """Raw launch: bf16((out * gain[h]) * bf16(sigmoid(gate))) as [B,N,H*64]; out bf16 [B,H,N,64], gain fp32
     [H], gate bf16 [B,N,H*64]."""
     _check_gate(out, gain, gate)
+    return _gate_forward(out, gain, gate)
+
+
+def _gate_forward(out, gain, gate):
     lib = _lib.load()
     B, H, N, hd = out.shape
     gated = torch.empty((B, N, H * hd), device=out.device, dtype=out.dtype)
@@ -118,6 +122,10 @@ def head_gate_backward(dgated, out, gain, gate, dgate, *, lse=None, query_start=
     of the [B,H,N] (delta, lse) pairs to write as well, 0 for none."""
     _check_gate(out, gain, gate, dgated, dgate)
     _expect(not pairs or (lse.shape == out.shape[:3] and lse.dtype == torch.float32), "lse fp32 [B,H,N] for the pairs")
+    return _gate_backward(dgated, out, gain, gate, dgate, lse, query_start, pairs)
+
+
+def _gate_backward(dgated, out, gain, gate, dgate, lse, query_start, pairs):
     lib = _lib.load()
     dout = torch.empty_like(out)
     dgain = torch.empty(gain.shape, device=out.device, dtype=torch.float32)
@@ -177,7 +185,7 @@ def block_forward(qkvg, pos_bias, scale_embed, phase_base, phase_gain, query_pro
     out = torch.empty((B, N, heads, HEAD_DIM), device=qkvg.device, dtype=qkvg.dtype)
     _, lse, y = dsqg_forward(*t, j_small, j_large, plane_shift, query_start, schedule=schedule,
                              query_probes=_planes(query_probes.float()), out=out.permute(0, 2, 1, 3))
-    gated = head_gate_forward(out.permute(0, 2, 1, 3), gain.float().contiguous(), gate)
+    gated = _gate_forward(out.permute(0, 2, 1, 3), gain.float().contiguous(), gate)
     return gated, out, lse, y, z
 
 
@@ -187,8 +195,9 @@ def block_backward(dgated, qkvg, pos_bias, scale_embed, phase_base, phase_gain, 
     _check_block(qkvg, gain, heads)
     B, N = qkvg.shape[:2]
     _expect(out.shape == (B, N, heads, HEAD_DIM) and dgated.shape == (B, N, heads * HEAD_DIM)
-            and lse.shape == (B, heads, N) and y.shape == z.shape == (B, heads, N, 4),
-            "out [B,N,H,64], dgated [B,N,H*64], lse [B,H,N] and y, z [B,H,N,4]")
+            and out.dtype == torch.bfloat16 and lse.shape == (B, heads, N) and lse.dtype == torch.float32
+            and y.shape == z.shape == (B, heads, N, 4),
+            "out bf16 [B,N,H,64], dgated [B,N,H*64], lse fp32 [B,H,N] and y, z [B,H,N,4]")
     qkvg = qkvg if qkvg.is_contiguous() and _rows_ok(qkvg) else qkvg.clone(memory_format=torch.contiguous_format)
     D = qkvg.shape[-1] // 4
     dgated = dgated.to(qkvg.dtype)
@@ -205,7 +214,7 @@ def block_backward(dgated, qkvg, pos_bias, scale_embed, phase_base, phase_gain, 
 
     def gate_launch(pairs):
         nonlocal dgain
-        dout, dgain = head_gate_backward(dgated, o, gain, gate, dgate, lse=lse, query_start=query_start, pairs=pairs)
+        dout, dgain = _gate_backward(dgated, o, gain, gate, dgate, lse, query_start, pairs)
         return dout
 
     g = dsqg_backward(gate_launch, *t, o, lse, j_small, j_large, plane_shift, query_start, schedule=schedule,
@@ -275,18 +284,19 @@ class _DSQGBlockFn(torch.autograd.Function):
         return grads + (None,) * 10
 
 
-def _plain_linear(m) -> bool:
-    """An nn.Linear nothing hooks into, of whole 16-byte rows and plain parameters: its forward is F.linear on its
-    weight and bias.  Hooks of its own, hooks on every module and a forward set on the instance (module trackers,
-    adapters, offloading) need the call, and so does a weight or bias of a class of its own."""
+def _plain_linear(m):
+    """(weight, bias) of an nn.Linear nothing hooks into, of whole 16-byte rows and plain parameters, whose forward is
+    F.linear on them; else None.  Hooks of its own, hooks on every module and a forward set on the instance (module
+    trackers, adapters, offloading) need the call, and so does a weight or bias of a class of its own."""
     every = torch.nn.modules.module
-    return (type(m) is torch.nn.Linear and m.in_features % 8 == 0 and m.out_features % 8 == 0
-            and not m._forward_pre_hooks and not m._forward_hooks
-            and not m._backward_hooks and not m._backward_pre_hooks
-            and not (every._global_forward_pre_hooks or every._global_forward_hooks
-                     or every._global_backward_hooks or every._global_backward_pre_hooks)
-            and "forward" not in m.__dict__
-            and all(p is None or type(p) in (torch.nn.Parameter, torch.Tensor) for p in (m.weight, m.bias)))
+    if (type(m) is not torch.nn.Linear or m.in_features % 8 or m.out_features % 8
+            or m._forward_pre_hooks or m._forward_hooks or m._backward_hooks or m._backward_pre_hooks
+            or every._global_forward_pre_hooks or every._global_forward_hooks
+            or every._global_backward_hooks or every._global_backward_pre_hooks or "forward" in m.__dict__):
+        return None
+    w, b = m.weight, m.bias
+    plain = (torch.nn.Parameter, torch.Tensor)
+    return (w, b) if type(w) in plain and (b is None or type(b) in plain) else None
 
 
 def _one_node(block, x: torch.Tensor) -> bool:
@@ -296,17 +306,17 @@ def _one_node(block, x: torch.Tensor) -> bool:
         return False
     if torch.is_grad_enabled() and (block.query_probes.requires_grad or block.key_probes.requires_grad):
         return False
-    proj, out, D = block.qkvg_proj, block.out_proj, block.num_heads * HEAD_DIM
-    if not (_plain_linear(proj) and _plain_linear(out)):
+    proj, out, gain, D = block.qkvg_proj, block.out_proj, block.if_gain, block.num_heads * HEAD_DIM
+    given, taken = _plain_linear(proj), _plain_linear(out)
+    if given is None or taken is None or x.dtype not in _AUTOCAST_TYPES:
         return False
-    # what autocast casts; float64 it leaves as it is, for the projections to keep or to refuse
-    if any(t is not None and t.dtype not in _AUTOCAST_TYPES for t in (x, proj.weight, proj.bias, out.weight, out.bias)):
-        return False
+    for t in (*given, *taken):
+        # what autocast casts; float64 it leaves as it is, for the projections to keep or to refuse
+        if t is not None and (t.dtype not in _AUTOCAST_TYPES or t.device != x.device):
+            return False
     return (block.head_dim == HEAD_DIM
             and proj.in_features == x.shape[-1] == D and proj.out_features == 4 * D and out.in_features == D
-            and all(t is None or t.device == x.device
-                    for t in (proj.weight, proj.bias, out.weight, out.bias, block.if_gain))
-            and block.if_gain.dtype == torch.float32 and block.if_gain.numel() == block.num_heads
+            and gain.dtype == torch.float32 and gain.numel() == block.num_heads and gain.device == x.device
             and str(block.backend).lower() in ("auto", "triton", "hip"))
 
 
